@@ -49,6 +49,9 @@ SIGNATURES = {
                                              c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p]),
     "eimoe_gemm_down_w8a8": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int,
                                      c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "eimoe_experts_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "eimoe_experts": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
+                              c_void_p, c_int, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),
     "eimoe_grouped_gemm": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_longlong, c_int,
                                    c_int,
                                    c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p]),

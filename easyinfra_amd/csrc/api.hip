@@ -291,8 +291,9 @@ int run_gate_up(const void* a, const int32_t* a_rows, long long a_nrows, int lda
 
 int run_down(const void* h, int I, const void* w, int w_dtype, const float* w_scale, int H, const int32_t* seg,
              int n_seg, int e_mod, int max_rows, void* y, int y_dtype, int k_split, int tile, hipStream_t s,
-             const float* h_scale = nullptr, int rows_hint = 0) {
+             const float* h_scale = nullptr, int rows_hint = 0, const int32_t* c_rows = nullptr) {
   GemmArgs p{};
+  p.c_rows = c_rows;
   p.rows_hint = rows_hint;
   p.a = h;
   p.a_rows = nullptr;
@@ -745,6 +746,112 @@ int eimoe_fused_moe_down_split(int T, int H, int I, int E, int k, int n_local, i
                                int flags) {
   if (T < 0 || H < 1 || I < 1 || k < 1 || n_local < 1 || shared_inter < 0) return 0;
   return fused_layout(T, H, I, E, k, n_local, shared_inter, out_dtype, flags).k_split;
+}
+
+}  // extern "C"
+
+namespace {
+
+struct ExpertsLayout {
+  size_t offsets, rows, pos, h, y, total;
+  int k_split;
+  bool planes;   // the down projection writes fp32 planes that the combine sums and reorders
+};
+
+// The down projection writes its rows straight to their places, except where a K split pays (experts
+// too large for the caches, >= 32 MiB, whose few-row launches need it to fill the GPU) and for fp32
+// experts of several ranks (whose kernel has no row map).
+ExpertsLayout experts_layout(int M, int H, int I, int H_out, int n_seg, int n_local, int w_dtype) {
+  ExpertsLayout L{};
+  const double expert_bytes = static_cast<double>(H_out) * I * elem_size(w_dtype);
+  L.k_split = expert_bytes >= 32.0 * 1024 * 1024 ? pick_down_split(M, 0, n_local, H_out, I, 4, false) : 1;
+  L.planes = L.k_split > 1 || (w_dtype == EIMOE_F32 && n_seg > n_local);
+  size_t o = 0;
+  auto take = [&](size_t bytes) {
+    const size_t at = o;
+    o += align256(bytes);
+    return at;
+  };
+  const size_t rows = static_cast<size_t>(M);
+  L.offsets = take(static_cast<size_t>(n_local + 1) * 4);
+  L.rows = take(rows * 4);
+  L.pos = take(rows * 4);
+  L.h = take(rows * I * (w_dtype == EIMOE_F32 ? 4 : 2));
+  if (L.planes) L.y = take(rows * H_out * 4 * L.k_split);
+  L.total = o;
+  return L;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t eimoe_experts_workspace_bytes(int M, int H, int I, int H_out, int n_seg, int n_local, int w_dtype) {
+  if (M < 0 || H < 1 || I < 1 || H_out < 1 || n_seg < 1 || n_local < 1 || elem_size(w_dtype) == 0) return 0;
+  return experts_layout(M, H, I, H_out, n_seg, n_local, w_dtype).total;
+}
+
+int eimoe_experts(const void* x, int M, int H, int I, int H_out, const void* w_gate_up, const void* w_down,
+                  int w_dtype, const float* w_gate_up_scale, const float* w_down_scale, const int32_t* counts,
+                  int n_seg, int n_local, void* y, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_gemm_common(M, n_seg, n_local);
+  if (rc) return rc;
+  if (n_seg % n_local) return fail(EIMOE_ERR_SHAPE, "n_seg=%d not a multiple of n_local=%d", n_seg, n_local);
+  if (w_dtype != EIMOE_BF16 && w_dtype != EIMOE_FP8 && w_dtype != EIMOE_F32)
+    return fail(EIMOE_ERR_DTYPE, "w_dtype=%d", w_dtype);
+  if (H < 64 || H % 64) return fail(EIMOE_ERR_ALIGN, "H=%d must be a positive multiple of 64", H);
+  if (I < 64 || I % 64) return fail(EIMOE_ERR_ALIGN, "I=%d must be a positive multiple of 64", I);
+  if (H_out < 64 || H_out % 64) return fail(EIMOE_ERR_ALIGN, "H_out=%d must be a positive multiple of 64", H_out);
+  const long long ab = w_dtype == EIMOE_F32 ? 4 : 2;
+  if (static_cast<long long>(M) * H * ab > 0x7fffffffll)
+    return fail(EIMOE_ERR_SHAPE, "x (%d rows x %d) exceeds 2 GiB", M, H);
+  if (static_cast<long long>(M) * I * ab > 0x7fffffffll)
+    return fail(EIMOE_ERR_SHAPE, "h (%d rows x %d) exceeds 2 GiB", M, I);
+  if (2ll * I * H * elem_size(w_dtype) > 0x7fffffffll)
+    return fail(EIMOE_ERR_SHAPE, "one expert's gate/up weights exceed 2 GiB");
+  if (static_cast<long long>(H_out) * I * elem_size(w_dtype) > 0x7fffffffll)
+    return fail(EIMOE_ERR_SHAPE, "one expert's down weights exceed 2 GiB");
+  if (M == 0) return EIMOE_OK;
+  REQUIRE_PTR(x);
+  REQUIRE_PTR(w_gate_up);
+  REQUIRE_PTR(w_down);
+  REQUIRE_PTR(counts);
+  REQUIRE_PTR(y);
+  REQUIRE_PTR(workspace);
+  if (w_dtype == EIMOE_FP8) {
+    REQUIRE_PTR(w_gate_up_scale);
+    REQUIRE_PTR(w_down_scale);
+  }
+  const ExpertsLayout L = experts_layout(M, H, I, H_out, n_seg, n_local, w_dtype);
+  if (workspace_bytes < L.total)
+    return fail(EIMOE_ERR_WORKSPACE, "workspace %zu bytes < required %zu", workspace_bytes, L.total);
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  auto at = [&](size_t off) { return static_cast<void*>(ws + off); };
+  const hipStream_t s = S(stream);
+  int32_t* offsets = static_cast<int32_t*>(at(L.offsets));
+  int32_t* rows = static_cast<int32_t*>(at(L.rows));
+  int32_t* pos = static_cast<int32_t*>(at(L.pos));
+  // one source rank: the rows are grouped by expert already
+  const bool merged = n_seg > n_local;
+  if (merged || L.planes) {
+    if ((rc = hip_check(launch_merge_segments(counts, n_seg, n_local, M, offsets, rows, pos, s), "merge segments")))
+      return rc;
+  } else if ((rc = hip_check(launch_counts_to_offsets(counts, n_seg, offsets, s), "counts_to_offsets"))) {
+    return rc;
+  }
+  if ((rc = run_gate_up(x, merged ? rows : nullptr, M, H, w_gate_up, w_dtype, w_gate_up_scale, H, I, offsets, n_local,
+                        n_local, M, at(L.h), EIMOE_TILE_AUTO, s)))
+    return rc;
+  const int y_dtype = w_dtype == EIMOE_F32 ? EIMOE_F32 : EIMOE_BF16;
+  if (!L.planes)
+    return run_down(at(L.h), I, w_down, w_dtype, w_down_scale, H_out, offsets, n_local, n_local, M, y, y_dtype, 1,
+                    EIMOE_TILE_AUTO, s, nullptr, 0, merged ? rows : nullptr);
+  if ((rc = run_down(at(L.h), I, w_down, w_dtype, w_down_scale, H_out, offsets, n_local, n_local, M, at(L.y),
+                     EIMOE_F32, L.k_split, EIMOE_TILE_AUTO, s)))
+    return rc;
+  return hip_check(launch_combine(at(L.y), EIMOE_F32, L.k_split, static_cast<long long>(M) * H_out, pos, nullptr, M, 1,
+                                  H_out, nullptr, 0, 1, y, y_dtype, s),
+                   "plane sum");
 }
 
 }  // extern "C"

@@ -404,6 +404,21 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, const TileCoord& tc,
   const auto& cs = sc.cs;
   const auto& cs_up = sc.cs_up;
   const auto& rs = sc.rs;
+  // the output rows, all loaded before the first store (see EpiScales)
+  int out_row[EPI == kEpiStoreBF16 ? MBE : 1][4];
+  if constexpr (EPI == kEpiStoreBF16) {
+#pragma unroll
+    for (int i = 0; i < MBE; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        out_row[i][r] = min(tc.row0 + wm * 16 * MBE + i * 16 + lq * 4 + r, tc.row_end - 1);
+    if (p.c_rows) {
+#pragma unroll
+      for (int i = 0; i < MBE; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) out_row[i][r] = p.c_rows[out_row[i][r]];
+    }
+  }
 #pragma unroll
   for (int i = 0; i < MBE; ++i) {
 #pragma unroll
@@ -433,8 +448,9 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, const TileCoord& tc,
         float v[G::NI];
 #pragma unroll
         for (int j = 0; j < G::NI; ++j) v[j] = acc[i][j][r] * rs[i][r] * cs[j];
+        const int c_row = EPI == kEpiStoreBF16 ? out_row[EPI == kEpiStoreBF16 ? i : 0][r] : row;
         const long long off =
-            static_cast<long long>(tc.split) * p.c_split_stride + static_cast<long long>(row) * p.ldc + col0;
+            static_cast<long long>(tc.split) * p.c_split_stride + static_cast<long long>(c_row) * p.ldc + col0;
         if constexpr (EPI == kEpiStoreF32) {
 #pragma unroll
           for (int g = 0; g < G::NI / G::CH; ++g)

@@ -31,6 +31,7 @@ struct GemmArgs {
   int S;
   int e_mod;
   void* c;
+  const int32_t* c_rows;     // bf16 store epilogue: row r of the product goes to row c_rows[r] of c; may be null
   void* c_lo;                // SiLU epilogue: also store bf16(h - bf16(h)) here (same layout as c); may be null
   long long ldc;
   long long c_split_stride;  // elements between split-K partial outputs
@@ -88,6 +89,10 @@ hipError_t launch_route_align(const float* logits, int T, int E, int k, int reno
                               int32_t* ids, float* w, int32_t* counts, int32_t* offsets, int32_t* sorted_flat,
                               int32_t* sorted_tok, int32_t* pos, int32_t* hist, hipStream_t s);
 hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offsets, hipStream_t s);
+// Segments (source rank, expert) regrouped by expert: merged bounds, merged -> original row and back
+// (S <= kMaxSeg, a multiple of n_exp; rows and pos hold max_rows entries).
+hipError_t launch_merge_segments(const int32_t* counts, int S, int n_exp, int max_rows, int32_t* offsets,
+                                 int32_t* rows, int32_t* pos, hipStream_t s);
 // MoE prologue: residual add + RMSNorm (+ router logits).  Routers of at most
 // kPrologueFusedMaxE experts and kPrologueFusedMaxGate bytes of gate weights are dotted in
 // the same pass; others (E % 64 == 0) go through the grouped GEMM with the T rows as one
@@ -109,7 +114,7 @@ hipError_t launch_moe_prologue(const void* hidden, const void* residual, const v
 
 hipError_t launch_gather_rows(const void* x, int row_bytes, const int32_t* rows, const int32_t* num_rows,
                               int max_rows, void* xs, hipStream_t s);
-// shared_n: planes of shared_y, T*H elements apart, summed (1 for a single plane).
+// shared_n: planes of shared_y, T*H elements apart, summed (1 for a single plane).  w null: weights 1.
 hipError_t launch_combine(const void* y, int y_dtype, int n_split, long long split_stride, const int32_t* pos,
                           const float* w, int T, int k, int H, const void* shared_y, int shared_dtype, int shared_n,
                           void* out, int out_dtype, hipStream_t s);

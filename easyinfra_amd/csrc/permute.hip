@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const void* __restrict__ y
     for (int j = 0; j < k; ++j) {
       const int p = pos[static_cast<long long>(t) * k + j];
       if (p < 0) continue;
-      const float wj = w[static_cast<long long>(t) * k + j];
+      const float wj = w ? w[static_cast<long long>(t) * k + j] : 1.f;
       float ys[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) ys[q] = 0.f;
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void combine_fixed_kernel(const void* __restri
 #pragma unroll
     for (int j = 0; j < K; ++j) {
       p[j] = pos[static_cast<long long>(t) * K + j];
-      wj[j] = w[static_cast<long long>(t) * K + j];
+      wj[j] = w ? w[static_cast<long long>(t) * K + j] : 1.f;
     }
     float v[K][NS][8];
 #pragma unroll

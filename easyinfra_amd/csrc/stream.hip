@@ -323,6 +323,14 @@ __global__ void __launch_bounds__(64 * W) grouped_gemm_stream_kernel(GemmArgs p)
   for (int m = 0; m < MBLK; ++m)
 #pragma unroll
     for (int r = 0; r < 4; ++r) rsv[m][r] = A8 ? p.a_scale[src_row[m][r]] : 1.f;
+  int out_row[MBLK][4];
+#pragma unroll
+  for (int m = 0; m < MBLK; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = min(row0 + m * 16 + lq * 4 + r, row_end - 1);
+      out_row[m][r] = EPI == kEpiStoreBF16 && p.c_rows ? p.c_rows[row] : row;
+    }
 #pragma unroll
   for (int m = 0; m < MBLK; ++m) {
 #pragma unroll
@@ -346,7 +354,7 @@ __global__ void __launch_bounds__(64 * W) grouped_gemm_stream_kernel(GemmArgs p)
         for (int f = 0; f < NFRAG; ++f) {
           const int col = col0 + f * 16 + lr;
           const long long off =
-              static_cast<long long>(split) * p.c_split_stride + static_cast<long long>(row) * p.ldc + col;
+              static_cast<long long>(split) * p.c_split_stride + static_cast<long long>(out_row[m][r]) * p.ldc + col;
           const float v = acc[m][f][r] * rs * cs[f];
           if constexpr (EPI == kEpiStoreF32) static_cast<float*>(p.c)[off] = v;
           else static_cast<uint16_t*>(p.c)[off] = f32_to_bf16(v);

@@ -9,8 +9,9 @@ arguments, the same parameters (``experts_gate_up_weight[E,2I,H]`` with gate row
 (source rank, local expert), output unweighted (the block applies routing weights
 at combine, moe_all2all.py:84, 291-307), empty input returned as is.
 
-The expert compute is two C-ABI grouped GEMMs (gate/up with SiLU*mul fused, then
-down); segment offsets come from the counts on the device, so no host sync.  For
+The expert compute is one C-ABI call: the rows of each expert gathered from every
+source rank into one segment (bounds from the counts on the device, so no host
+sync), then two grouped GEMMs (gate/up with SiLU*mul fused, then down).  For
 the whole layer (routing included) see ``forward_layer`` / ``easyinfra_amd.fused_moe``.
 """
 from __future__ import annotations
@@ -129,13 +130,8 @@ class HipFusedMoE(nn.Module):
             return hidden_states
         x = hidden_states if hidden_states.is_contiguous() else hidden_states.contiguous()
         counts = self._counts_tensor(expert_count, x.device)
-        offsets = ops.counts_to_offsets(counts)
-        M = x.shape[0]
-        E = self.num_physical_experts
-        s_gu, s_d = self.w_scales if self.w_scales is not None else (None, None)
-        h = ops.gemm_gate_up_silu(x, self.experts_gate_up_weight, offsets, M, w_scale=s_gu, e_mod=E)
-        y = ops.gemm_down(h, self.experts_down_weight, offsets, M, out_dtype=x.dtype, w_scale=s_d, e_mod=E)
-        return y[0]
+        return ops.experts(x, self.experts_gate_up_weight, self.experts_down_weight, counts,
+                           self.num_physical_experts, self.w_scales)
 
     def forward_noep(self, hidden_states: torch.Tensor, expert_count: Union[torch.Tensor, Sequence[int]]):
         """ep=1: the same grouped expert compute (rows grouped by local expert)."""

@@ -323,6 +323,39 @@ def gemm_down_w8a8(hq: torch.Tensor, h_scale: torch.Tensor, w_down: torch.Tensor
     return y
 
 
+def experts(x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, counts: torch.Tensor, n_local: int,
+            w_scales: Optional[Tuple[torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
+    """fused_moe.py:106-156 on pre-grouped rows: the n_local experts' MLP, unweighted; x holds counts[s] rows
+    of segment s = rank * n_local + e one after the other -> y [M, H] in x's order and dtype."""
+    f32 = w_gate_up.dtype == torch.float32
+    _req(x, "x", torch.float32 if f32 else torch.bfloat16, 2)
+    _req(w_gate_up, "w_gate_up", (torch.bfloat16, torch.float8_e4m3fn, torch.float32), 3)
+    _req(w_down, "w_down", w_gate_up.dtype, 3)
+    _req(counts, "counts", torch.int32, 1)
+    E, I2, H = w_gate_up.shape
+    H_out, I = w_down.shape[1], w_down.shape[2]
+    if x.shape[1] != H:
+        raise ValueError(f"x has {x.shape[1]} columns, weights expect H={H}")
+    if I2 != 2 * I:
+        raise ValueError(f"h has {I2 // 2} columns, weights expect I={I}")
+    if min(E, w_down.shape[0]) < n_local:
+        raise ValueError(f"weights hold {min(E, w_down.shape[0])} experts, {n_local} expected")
+    if (w_scales is not None) != (w_gate_up.dtype == torch.float8_e4m3fn):
+        raise ValueError("fp8 weights need w_scales=(s_gate_up [E, 2I], s_down [E, H]); bf16 weights take none")
+    s_gu, s_d = w_scales if w_scales is not None else (None, None)
+    if w_scales is not None:
+        _req_shape(s_gu, "w_scales[0] (gate/up)", (E, I2))
+        _req_shape(s_d, "w_scales[1] (down)", (w_down.shape[0], H_out))
+    M = x.shape[0]
+    dt = _dt(w_gate_up)
+    need = int(_lib.lib().eimoe_experts_workspace_bytes(M, H, I, H_out, counts.numel(), n_local, dt))
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
+    y = torch.empty(M, H_out, dtype=x.dtype, device=x.device)
+    call("eimoe_experts", x.data_ptr(), M, H, I, H_out, w_gate_up.data_ptr(), w_down.data_ptr(), dt, _ptr(s_gu),
+         _ptr(s_d), counts.data_ptr(), counts.numel(), n_local, y.data_ptr(), ws.data_ptr(), need, _stream(x))
+    return y
+
+
 def grouped_gemm(a: torch.Tensor, b: torch.Tensor, seg_offsets: torch.Tensor, max_rows: int,
                  out_dtype=torch.bfloat16, a_rows: Optional[torch.Tensor] = None,
                  b_scale: Optional[torch.Tensor] = None, e_mod: Optional[int] = None, tile: int = 0) -> torch.Tensor:

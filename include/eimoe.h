@@ -184,6 +184,18 @@ int eimoe_gemm_down_w8a8(const void* hq, const float* h_scale, int I, const void
                          const int32_t* seg_offsets, int n_seg, int e_mod, int max_rows, void* y, int y_dtype,
                          int k_split, int tile, void* stream);
 
+/* The experts' MLP on pre-grouped rows: FusedMoE.forward_ep(hidden_states, expert_count)
+ * (fused_moe.py:106-156), unweighted.  x [M, H] holds the rows of segment s = rank * n_local + e one
+ * after the other, counts[s] each (device int32, n_seg a multiple of n_local); y [M, H_out] keeps
+ * their order.  Rows of one expert from several source ranks are computed as one segment, so its
+ * weights are read once.  w_gate_up [n_local, 2I, H], w_down [n_local, H_out, I]: bf16 or fp8 (with
+ * channel scales) and x, y bf16; or all fp32.  h is rounded to bf16 (fp32 experts: fp32), y once from
+ * the fp32 sums.  H, I, H_out multiples of 64.  workspace: eimoe_experts_workspace_bytes bytes. */
+size_t eimoe_experts_workspace_bytes(int M, int H, int I, int H_out, int n_seg, int n_local, int w_dtype);
+int eimoe_experts(const void* x, int M, int H, int I, int H_out, const void* w_gate_up, const void* w_down,
+                  int w_dtype, const float* w_gate_up_scale, const float* w_down_scale, const int32_t* counts,
+                  int n_seg, int n_local, void* y, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Plain grouped GEMM, the X_grouped_gemm_single(A, B_list, block_sizes) contract
  * (single_group_gemm_moe.py:76-91): c[rows_s] = a[rows_s] . B[s % e_mod]^T with B packed as
  * [E_w, N, K] (b_expert_stride elements apart).  a bf16 [a_nrows, lda] (rows gathered through a_rows

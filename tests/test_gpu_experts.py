@@ -1,0 +1,74 @@
+"""The experts' MLP on pre-grouped rows (eimoe_experts): rows of one expert from several source ranks
+computed as one segment, written back in their own order, against the oracle per segment."""
+import pytest
+import torch
+
+import oracle
+from easyinfra_amd import _lib, ops
+
+
+def test_experts_validation():
+    f = _lib.lib().eimoe_experts
+    ok = dict(x=1, M=8, H=128, I=128, Ho=128, gu=1, d=1, dt=_lib.BF16, sg=None, sd=None, c=1, S=8, E=4, y=1, ws=1,
+              wsb=1 << 30, st=None)
+    rc = lambda **kw: f(*dict(ok, **kw).values())
+    assert rc(S=6) == _lib.ERR_SHAPE                      # segments not a multiple of the experts
+    assert rc(S=2000, E=2) == _lib.ERR_SHAPE              # too many segments
+    assert rc(H=100) == _lib.ERR_ALIGN and rc(I=96) == _lib.ERR_ALIGN and rc(Ho=32) == _lib.ERR_ALIGN
+    assert rc(dt=7) == _lib.ERR_DTYPE
+    assert rc(dt=_lib.FP8) == _lib.ERR_NULL               # fp8 without scales
+    assert rc(c=None) == _lib.ERR_NULL
+    assert rc(wsb=16) == _lib.ERR_WORKSPACE
+    assert rc(M=1 << 20, H=1024) == _lib.ERR_SHAPE        # x: 2 GiB
+    assert rc(M=0, x=None) == _lib.EIMOE_OK
+
+
+# (experts, ranks, H, I, counts): one row, empty segments and ranks, tile edges (16, 32, 64, 128, 256
+# rows and one past), one hot expert, more segments than the register tile schedule holds (64 experts
+# on one rank against 65), and an expert of 32 MiB (K split planes).
+def _counts(E, ep, pattern, seed):
+    g = torch.Generator().manual_seed(seed)
+    c = torch.zeros(ep, E, dtype=torch.int64)
+    if pattern == "one":
+        c[ep - 1, E // 2] = 1
+    elif pattern == "edges":
+        v = [0, 1, 15, 16, 17, 31, 33, 64, 65, 0, 127, 129]
+        for i in range(ep * E):
+            c.view(-1)[i] = v[i % len(v)]
+    elif pattern == "hot":
+        c[:, 0] = 300
+        c[0, E - 1] = 2
+    else:
+        c = torch.randint(0, 12, (ep, E), generator=g)
+    return c
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,ep,H,I,pattern", [(4, 1, 128, 128, "edges"), (4, 2, 128, 192, "one"), (5, 3, 192, 128, "edges"),
+                                              (3, 4, 256, 256, "hot"), (1, 8, 128, 128, "edges"), (65, 2, 128, 64, "few"),
+                                              (64, 16, 64, 64, "few"), (2, 2, 1024, 16384, "few")])
+@pytest.mark.parametrize("mode", ["bf16", "w8a16", "fp32"])
+def test_experts_match_oracle_per_segment(dev, E, ep, H, I, pattern, mode):
+    g = torch.Generator().manual_seed(E * ep + I)
+    counts = _counts(E, ep, pattern, E)
+    M = int(counts.sum())
+    dt = torch.float32 if mode == "fp32" else torch.bfloat16
+    x = torch.randn(M, H, generator=g).to(dt)
+    wgu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(dt)
+    wd = (torch.randn(E, H, I, generator=g) * 0.05).to(dt)
+    ref_gu, ref_d, scales = wgu.float(), wd.float(), None
+    if mode == "w8a16":
+        (wgu, sgu), (wd, sd) = oracle.quantize_weights_fp8(wgu.float()), oracle.quantize_weights_fp8(wd.float())
+        ref_gu, ref_d = wgu.float() * sgu[..., None], wd.float() * sd[..., None]
+        scales = (sgu.to(dev), sd.to(dev))
+    print("CASE", dict(E=E, ep=ep, H=H, I=I, pattern=pattern, mode=mode, M=M), flush=True)
+    y = ops.experts(x.to(dev), wgu.to(dev), wd.to(dev), counts.reshape(-1).to(torch.int32).to(dev), E, scales)
+    assert y.shape == (M, H) and y.dtype == dt
+    ref, r = torch.empty(M, H), 0
+    for s, c in enumerate(counts.reshape(-1).tolist()):
+        ref[r:r + c] = oracle.expert_mlp(x[r:r + c].float(), ref_gu[s % E], ref_d[s % E], round_h_bf16=mode != "fp32")
+        r += c
+    # one bf16 rounding of the output (at most 2^-9 of each value) and h values whose bf16 rounding
+    # flips with the order of the fp32 sums (far fewer); W8A16 forms the oracle's products with the
+    # scale applied to the sum instead of the weight (fp32 rounding).  fp32: sums of up to 16384 terms.
+    assert oracle.rel_l2(y.cpu().float(), ref) <= (2e-5 if mode == "fp32" else 2.0 ** -8)
