@@ -146,11 +146,7 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
     // height, and routed segments scatter around the mean, so an expected count just past a
     // multiple of 256 rows gives about half the segments one more m-tile.  Count
     // E[ceil(rows / 256)] with the rows ~ normal(mean, sqrt(mean)).
-    const double sd = std::sqrt(std::max(per, 1.0));
-    double e = 0.0;
-    for (int j = 0; j * static_cast<double>(bm) < per + 6.0 * sd; ++j)
-      e += 0.5 * std::erfc((j * static_cast<double>(bm) + 0.5 - per) / (sd * std::sqrt(2.0)));
-    mt = segs * e;
+    mt = segs * expected_m_tiles(per, bm);
   } else {
     // m-tiles in full-tile units from the expected rows per segment: whole tiles plus the
     // remainder's tile, which takes a quarter, half or full height (a short tile costs its share)

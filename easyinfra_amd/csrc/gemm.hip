@@ -307,16 +307,100 @@ __device__ __forceinline__ void mma_f32(f32x4_t (&acc)[MBE][G::NB], const bf16x8
   }
 }
 
-// One 64-wide K slab: two 32-wide MFMA steps, each reading its fragments first.
-template <class G, int MBE, bool F32 = false>
+// fp32 operands as three bf16 terms on the bf16 MFMA: x = hi + mid + lo, each the upper half of what
+// the terms before it leave.  A fp32 mantissa has 24 bits and each term takes 8, so the three hold x
+// exactly (down to terms below 2^-133).  Lane group q's eight values of a 32-wide k slab are the
+// 16-byte chunks q and q + 4 of the row, for A and B alike.
+struct Split3 {
+  bf16x8_t t[3];   // hi, mid, lo
+};
+
+__device__ __forceinline__ Split3 split3(const f32x4_t& c0, const f32x4_t& c1) {
+  u32x4_t w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float x0 = i < 2 ? c0[2 * i] : c1[2 * i - 4];
+    float x1 = i < 2 ? c0[2 * i + 1] : c1[2 * i - 3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+      w[k][i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);   // the upper halves
+      x0 -= __uint_as_float(u0 & 0xffff0000u);
+      x1 -= __uint_as_float(u1 & 0xffff0000u);
+    }
+  }
+  return Split3{{__builtin_bit_cast(bf16x8_t, w[0]), __builtin_bit_cast(bf16x8_t, w[1]),
+                 __builtin_bit_cast(bf16x8_t, w[2])}};
+}
+
+__device__ __forceinline__ Split3 split3_lds(const uint16_t* s, int R, int q) {
+  return split3(*reinterpret_cast<const f32x4_t*>(&s[R * 64 + ((q ^ swz(R)) << 3)]),
+                *reinterpret_cast<const f32x4_t*>(&s[R * 64 + (((q + 4) ^ swz(R)) << 3)]));
+}
+
+// One row of fragments times all columns: the six products above 2^-22 of x*y, smallest first.
+template <int NB>
+__device__ __forceinline__ void mma_split3(f32x4_t (&acc)[NB], const Split3& a, const Split3 (&b)[NB]) {
+  constexpr int ta[6] = {2, 0, 1, 1, 0, 0};
+  constexpr int tb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.t[ta[k]], b[j].t[tb[k]], acc[j], 0, 0, 0);
+}
+
+// One 32-wide fp32 slab from the split terms.
+template <class G, int MBE>
+__device__ __forceinline__ void slab_mma_split3(f32x4_t (&acc)[MBE][G::NB], const uint16_t* sA, const uint16_t* sB,
+                                                int wm, int wn, int lane) {
+  const int lr = lane & 15;
+  const int q = lane >> 4;
+  Split3 b[G::NB];
+#pragma unroll
+  for (int j = 0; j < G::NB; ++j) b[j] = split3_lds(sB, wn * G::WN + j * 16 + lr, q);
+#pragma unroll
+  for (int i = 0; i < MBE; ++i) mma_split3<G::NB>(acc[i], split3_lds(sA, wm * 16 * MBE + i * 16 + lr, q), b);
+}
+
+// Whether the split terms may not stand for a tile's operands, told from its sums: one is infinite or
+// NaN, or nonzero below 2^-64 (operands below 2^-109 reach past the smallest bf16, 2^-133, before their
+// 24 bits end; ordinary sums that small are cancellations of about one in 10^18).
+template <class G, int MBE>
+__device__ __forceinline__ bool split3_doubtful(const f32x4_t (&acc)[MBE][G::NB]) {
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < MBE; ++i)
+#pragma unroll
+    for (int j = 0; j < G::NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float m = fabsf(acc[i][j][r]);
+        bad |= !(m <= 3.4028234663852886e38f) | ((m < 0x1p-64f) & (m != 0.f));
+      }
+  return bad;
+}
+
+// What a slab's MFMAs take: bf16 operands, fp32 operands on the fp32 MFMA, fp32 operands split.
+enum SlabOps : int { kSlabBF16 = 0, kSlabF32 = 1, kSlabSplit3 = 2 };
+// fp32 tiles of at least this many rows take the split terms; below, the fp32 MFMA.
+constexpr int kSplit3MinRows = 32;
+
+// One 128-byte K slab (64 bf16 or 32 fp32): two MFMA steps, each reading its fragments first, or one
+// of the split terms.
+template <class G, int MBE, int OPS = kSlabBF16>
 __device__ __forceinline__ void slab_mma(f32x4_t (&acc)[MBE][G::NB], const uint16_t* sA, const uint16_t* sB, int wm,
                                          int wn, int lane) {
+  if constexpr (OPS == kSlabSplit3) {
+    slab_mma_split3<G, MBE>(acc, sA, sB, wm, wn, lane);
+  } else {
 #pragma unroll
-  for (int kk = 0; kk < G::BK / 32; ++kk) {
-    bf16x8_t af[MBE], bfr[G::NB];
-    read_frags<G, MBE>(sA, sB, kk, wm, wn, lane, af, bfr);
-    if constexpr (F32) mma_f32<G, MBE>(acc, af, bfr);
-    else mma<G, MBE>(acc, af, bfr);
+    for (int kk = 0; kk < G::BK / 32; ++kk) {
+      bf16x8_t af[MBE], bfr[G::NB];
+      read_frags<G, MBE>(sA, sB, kk, wm, wn, lane, af, bfr);
+      if constexpr (OPS == kSlabF32) mma_f32<G, MBE>(acc, af, bfr);
+      else mma<G, MBE>(acc, af, bfr);
+    }
   }
 }
 
@@ -671,29 +755,40 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_dma_kernel(GemmAr
   by_height<BM, G::MB, A_PW>(tc.row_end - tc.row0, [&]<int MBE>() {
     constexpr int A_CNT = A_PW * MBE / G::MB;
     f32x4_t acc[MBE][G::NB];
+    auto k_loop = [&]<int OPS>() {
 #pragma unroll
-    for (int i = 0; i < MBE; ++i)
+      for (int i = 0; i < MBE; ++i)
 #pragma unroll
-      for (int j = 0; j < G::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, 0, b_nt);
-    __syncthreads();
-    int kt = 0;
-    // Slab kt is in buffer 0 at the top of each iteration.  The second load is unconditional
-    // (on the last iteration of an even slab count it re-reads slab KT-1 into buffer 0, which is
-    // not read again and which the closing barrier waits for) so that it is not split into its
-    // own basic block, where the scheduler would queue the previous slab's MFMAs ahead of it.
-    for (; kt + 1 < KT; kt += 2) {
-      issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA1, sB1, wave, (kt + 1) * BK * 2, b_nt);
-      pin_issue();
-      slab_mma<G, MBE, F32>(acc, sA0, sB0, wm, wn, lane);
+        for (int j = 0; j < G::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, 0, b_nt);
       __syncthreads();
-      issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, min(kt + 2, KT - 1) * BK * 2,
-                                      b_nt);
-      pin_issue();
-      slab_mma<G, MBE, F32>(acc, sA1, sB1, wm, wn, lane);
-      __syncthreads();
+      int kt = 0;
+      // Slab kt is in buffer 0 at the top of each iteration.  The second load is unconditional
+      // (on the last iteration of an even slab count it re-reads slab KT-1 into buffer 0, which is
+      // not read again and which the closing barrier waits for) so that it is not split into its
+      // own basic block, where the scheduler would queue the previous slab's MFMAs ahead of it.
+      for (; kt + 1 < KT; kt += 2) {
+        issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA1, sB1, wave, (kt + 1) * BK * 2, b_nt);
+        pin_issue();
+        slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane);
+        __syncthreads();
+        issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, min(kt + 2, KT - 1) * BK * 2,
+                                        b_nt);
+        pin_issue();
+        slab_mma<G, MBE, OPS>(acc, sA1, sB1, wm, wn, lane);
+        __syncthreads();
+      }
+      if (kt < KT) slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane);   // odd slab count: last slab in buffer 0
+    };
+    if constexpr (F32 && BM >= kSplit3MinRows) {
+      // Infinite and NaN operands (and products past the fp32 range) leave sums that are not finite,
+      // as on the fp32 MFMA but not the same ones (inf * 0 among the split terms): such a tile is
+      // computed again on the fp32 MFMA.  The vote is also the barrier before the stages are reused.
+      k_loop.template operator()<kSlabSplit3>();
+      if (__syncthreads_or(split3_doubtful<G, MBE>(acc) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
+    } else {
+      k_loop.template operator()<F32 ? kSlabF32 : kSlabBF16>();
     }
-    if (kt < KT) slab_mma<G, MBE, F32>(acc, sA0, sB0, wm, wn, lane);   // odd slab count: last slab in buffer 0
     epilogue<G, EPI, MBE>(p, tc, acc, wm, wn, lane, nullptr, nullptr);
   });
 }
@@ -847,16 +942,41 @@ __device__ __forceinline__ void ring_frag_addrs(uint32_t aA, uint32_t aB, int wm
   }
 }
 
+// A slab's MFMAs from its fragments (both K halves: A then B of half 0, then of half 1).  For fp32 the
+// halves are the chunks q and q + 4 of each row, which the split takes as one 32-wide fragment.
+template <class G, int MBE, int OPS>
+__device__ __forceinline__ void ring_mma(f32x4_t (&acc)[MBE][G::NB], bf16x8_t (&fr)[2 * (MBE + G::NB)]) {
+  constexpr int F = MBE + G::NB;
+  if constexpr (OPS == kSlabSplit3) {
+    auto split = [&](int i) {
+      return split3(__builtin_bit_cast(f32x4_t, fr[i]), __builtin_bit_cast(f32x4_t, fr[F + i]));
+    };
+    Split3 b[G::NB];
+#pragma unroll
+    for (int j = 0; j < G::NB; ++j) b[j] = split(MBE + j);
+#pragma unroll
+    for (int i = 0; i < MBE; ++i) mma_split3<G::NB>(acc[i], split(i), b);
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      auto& af = *reinterpret_cast<bf16x8_t(*)[MBE]>(fr + kk * F);
+      auto& bfr = *reinterpret_cast<bf16x8_t(*)[G::NB]>(fr + kk * F + MBE);
+      if constexpr (OPS == kSlabF32) mma_f32<G, MBE>(acc, af, bfr);
+      else mma<G, MBE>(acc, af, bfr);
+    }
+  }
+}
+
 // grouped_gemm_dma_kernel on a ring of NS LDS stages: NS - 1 slabs in flight per workgroup instead
 // of one.  The two-stage loop's __syncthreads() fences wait for every DMA in flight at each slab
 // end; here each slab ends waiting for its wave's next slab only (loads complete in issue order)
 // and a barrier without a fence publishes it.  Same tiles, LDS layout per stage and accumulation
 // order: bit-identical results.  For launches whose tiles fit the GPU at the ring's occupancy.
-template <int BM, int BN, int WGM, int WGN, int EPI, int GM, int NS>
+template <int BM, int BN, int WGM, int WGN, int EPI, int GM, int NS, bool F32 = false>
 __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmArgs p) {
   static_assert(NS == 3, "three stages");
   using G = Geo<BM, BN, WGM, WGN, EPI>;
-  constexpr int EB = 2;
+  constexpr int EB = F32 ? 4 : 2;
   constexpr int BK = G::BK;
   constexpr int NW = G::NW;
   constexpr int A_PW = BM / 8 / G::NW;
@@ -901,19 +1021,20 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     constexpr int A_CNT = A_PW * MBE / G::MB;
     constexpr int L = A_CNT + B_PW;   // DMA instructions per slab per wave
     f32x4_t acc[MBE][G::NB];
-#pragma unroll
-    for (int i = 0; i < MBE; ++i)
-#pragma unroll
-      for (int j = 0; j < G::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // slabs 0 and 1 into stages 0 and 1 (clamped to the last slab: stages not read again)
-    issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, t0.a, t0.b, wave, 0, b_nt);
-    issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, t1.a, t1.b, wave, min(1, KT - 1) * BK * 2, b_nt);
-    wait_vm<(NS - 2) * L>();   // this wave's slab 0
-    pp_barrier();
     // slab kt + J: read stage J, load slab kt + J + NS - 1 into the stage slab kt + J - 1 read (every
     // wave finished reading it before the barrier that ended that slab).
     // The slab's DMA goes first, then its fragment reads and their wait (lds_read_wait), its MFMAs, and
     // the wait for the next slab's data.
+    auto k_loop = [&]<int OPS>() {
+#pragma unroll
+      for (int i = 0; i < MBE; ++i)
+#pragma unroll
+        for (int j = 0; j < G::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      // slabs 0 and 1 into stages 0 and 1 (clamped to the last slab: stages not read again)
+      issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, t0.a, t0.b, wave, 0, b_nt);
+      issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, t1.a, t1.b, wave, min(1, KT - 1) * BK * 2, b_nt);
+      wait_vm<(NS - 2) * L>();   // this wave's slab 0
+      pp_barrier();
 #define EIMOE_RING_SLAB(J, SA, SB, SAN, SBN)                                                                \
   if (kt + J < KT) {                                                                                        \
     issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, SAN, SBN, wave, min(kt + J + NS - 1, KT - 1) * BK * 2, \
@@ -922,19 +1043,24 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     ring_frag_addrs<G, MBE>(lds_addr(SA), lds_addr(SB), wm, wn, lane, ad);                                  \
     bf16x8_t fr[2 * (MBE + G::NB)];                                                                         \
     lds_read_wait(ad, fr);                                                                                  \
-    mma<G, MBE>(acc, *reinterpret_cast<bf16x8_t(*)[MBE]>(fr), *reinterpret_cast<bf16x8_t(*)[G::NB]>(fr + MBE)); \
-    mma<G, MBE>(acc, *reinterpret_cast<bf16x8_t(*)[MBE]>(fr + MBE + G::NB),                                 \
-                *reinterpret_cast<bf16x8_t(*)[G::NB]>(fr + 2 * MBE + G::NB));                               \
+    ring_mma<G, MBE, OPS>(acc, fr);                                                                         \
     wait_vm<(NS - 2) * L>();                                                                                \
     pp_barrier();                                                                                           \
   }
-    for (int kt = 0; kt < KT; kt += NS) {
-      EIMOE_RING_SLAB(0, t0.a, t0.b, t2.a, t2.b)
-      EIMOE_RING_SLAB(1, t1.a, t1.b, t0.a, t0.b)
-      EIMOE_RING_SLAB(2, t2.a, t2.b, t1.a, t1.b)
-    }
+      for (int kt = 0; kt < KT; kt += NS) {
+        EIMOE_RING_SLAB(0, t0.a, t0.b, t2.a, t2.b)
+        EIMOE_RING_SLAB(1, t1.a, t1.b, t0.a, t0.b)
+        EIMOE_RING_SLAB(2, t2.a, t2.b, t1.a, t1.b)
+      }
 #undef EIMOE_RING_SLAB
-    pp_wait_vm0();   // the clamped loads near the end land before the workgroup's LDS is released
+      pp_wait_vm0();   // the clamped loads near the end land before the workgroup's LDS is released (or reused)
+    };
+    if constexpr (F32 && BM >= kSplit3MinRows) {
+      k_loop.template operator()<kSlabSplit3>();   // as in grouped_gemm_dma_kernel
+      if (__syncthreads_or(split3_doubtful<G, MBE>(acc) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
+    } else {
+      k_loop.template operator()<F32 ? kSlabF32 : kSlabBF16>();
+    }
     epilogue<G, EPI, MBE>(p, tc, acc, wm, wn, lane, nullptr, nullptr);
   });
 }
@@ -1998,6 +2124,15 @@ static int lds_tile_wgs(int stage_bytes, int stages) {
   return 160 / kib;
 }
 
+// E[ceil(rows / bm)] of a segment whose rows scatter around their mean (normal, variance = mean).
+double expected_m_tiles(double rows, int bm) {
+  const double sd = std::sqrt(std::max(rows, 1.0));
+  double e = 0.0;
+  for (int j = 0; j * static_cast<double>(bm) < rows + 6.0 * sd; ++j)
+    e += 0.5 * std::erfc((j * static_cast<double>(bm) + 0.5 - rows) / (sd * std::sqrt(2.0)));
+  return e;
+}
+
 // stage_bytes: one stage of the tile (bf16: a 64-k slab of A and B; W8A16: a 128-k chunk of both).
 static bool use_ring_tile(const GemmArgs& p, int bm, int stage_bytes, int n_tiles) {
   const int S = p.S > 0 ? p.S : 1;
@@ -2326,6 +2461,20 @@ static hipError_t launch_cfg_f32(const GemmArgs& p, int max_rows, hipStream_t s)
   long long grid = (max_mt * n_tiles * p.k_split + kNumXcd - 1) / kNumXcd * kNumXcd;
   if (grid < kNumXcd) grid = kNumXcd;
   if (grid > 0x7fffffffll) return hipErrorInvalidValue;
+  // The ring where its workgroups hold all the expected tiles in one round (weights streamed at a few
+  // rows per expert: the tiny-Mixtral gate/up at 2 / 8 / 24 rows in all 27.3 / 30.0 / 35.5 -> 18.2 / 23.3 /
+  // 34.1 us on 16x64, its down projection with K split 4 20.0 / 20.9 / 23.2 -> 13.6 / 14.6 / 18.8); past
+  // one round the two-stage kernel's extra workgroups per CU win (512 rows on 64x128: 75.4 against 87.2).
+  if constexpr (BM <= 64) {
+    const int S = p.S > 0 ? p.S : 1;
+    const double avg = static_cast<double>(p.rows_hint > 0 ? std::min(p.rows_hint, p.max_rows) : p.max_rows) / S;
+    const double est = S * expected_m_tiles(avg, BM) * n_tiles * p.k_split;
+    if (est <= static_cast<double>(lds_tile_wgs((BM + BN) * 128, 3)) * kNumCu) {
+      hipLaunchKernelGGL((grouped_gemm_ring_kernel<BM, BN, WGM, WGN, EPI, GM, 3, true>),
+                         dim3(static_cast<unsigned>(grid)), dim3(WGM * WGN * 64), 0, s, p);
+      return hipGetLastError();
+    }
+  }
   hipLaunchKernelGGL((grouped_gemm_dma_kernel<BM, BN, WGM, WGN, EPI, GM, true>), dim3(static_cast<unsigned>(grid)),
                      dim3(WGM * WGN * 64), 0, s, p);
   return hipGetLastError();
@@ -2335,26 +2484,35 @@ template <int EPI>
 static hipError_t launch_epi_f32(const GemmArgs& p, int max_rows, int tile, hipStream_t s) {
   switch (tile) {
     case kTileM: return launch_cfg_f32<128, 128, 2, 2, EPI, 4>(p, max_rows, s);
+    case kTileMS: return launch_cfg_f32<64, 128, 2, 2, EPI, 4>(p, max_rows, s);
     case kTileS: return launch_cfg_f32<32, 128, 1, 4, EPI, 1>(p, max_rows, s);
     case kTileXS: return launch_cfg_f32<16, 64, 1, 2, EPI, 1>(p, max_rows, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-// The fp32 MFMA runs at 1/16 of the bf16 rate, so LDS and memory are far from the limit: the
-// 128x128 tile from 32 rows per segment, 32x128 and 16x64 below.
+// fp32 tiles.  16x64 multiplies on the fp32 MFMA (its few rows are bound by the weights), the taller
+// tiles split their operands into bf16 terms: six bf16 MFMAs cost 6/16 of the fp32 one.  By expected
+// rows per segment, measured on the tiny-Mixtral shape (8 experts, 1024 x 2816, cold, one box; us):
+// gate/up on 16x64 / 32x128 / 64x128 / 128x128 at 16 rows 37 / 40 / 40 / 50, at 24 rows 44 / 39 / 50 /
+// 54, at 32 rows 67 / 52 / 52 / 62, at 96 rows 123 / 98 / 80 / 84, at 128 rows 167 / 124 / 103 / 135, at
+// 256 rows 366 / 217 / 168 / 165, at 512 rows 776 / 407 / 298 / 295; down (K split 4) at 16 rows 20 / 21 /
+// 23 / 29, at 32 rows 27 / 26 / 29 / 33, at 64 rows 44 / 39 / 40 / 46, at 128 rows 68 / 60 / 55 / 62, at 256
+// rows 123 / 100 / 87 / 103.  The layer at 512 tokens: 251 -> 175 us against the fp32 MFMA on
+// 128x128, error against float64 9.9e-7 -> 8.7e-7; at 1 / 40 tokens 56 -> 44 / 68 -> 61 us.
 hipError_t launch_grouped_gemm_f32(const GemmArgs& p, int epi, int max_rows, int tile, hipStream_t s) {
   if (epi != kEpiSiluF32 && epi != kEpiStoreF32) return hipErrorInvalidValue;
   if (tile == kTileAuto) {
     const double avg = static_cast<double>(p.rows_hint > 0 ? std::min(p.rows_hint, p.max_rows) : p.max_rows) /
                        (p.S > 0 ? p.S : 1);
-    tile = avg >= 32 ? kTileM : avg >= 12 ? kTileS : kTileXS;
+    if (epi_silu(epi)) tile = avg < 18 ? kTileXS : avg < 30 ? kTileS : avg < 256 ? kTileMS : kTileM;
+    else tile = avg < 36 ? kTileXS : avg < 512 ? kTileMS : kTileM;
   }
-  // No 256x256, 64x128 or streaming fp32 kernel: those requests take the 128x128 tile.  Whatever
+  // No 256x256 or streaming fp32 kernel: those requests take the 128x128 tile.  Whatever
   // the start, step down until the tile's output columns divide N (the tile's columns are its
   // grid's only bound on N), and refuse a tile that still does not fit rather than leave columns
   // unwritten.
-  if (tile == kTileL || tile == kTileMS || tile == kTileStream) tile = kTileM;
+  if (tile == kTileL || tile == kTileStream) tile = kTileM;
   while (tile != kTileXS && p.N % gemm_out_cols_per_tile(tile, epi) != 0) tile = tile_step_down(tile);
   if (p.N % gemm_out_cols_per_tile(tile, epi) != 0) return hipErrorInvalidValue;
   return epi == kEpiSiluF32 ? launch_epi_f32<kEpiSiluF32>(p, max_rows, tile, s)

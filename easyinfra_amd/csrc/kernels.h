@@ -141,8 +141,10 @@ bool stream_gemm_supported(const GemmArgs& p, int epi, int ops);
 int stream_out_cols(int N, int epi, bool fp8);
 hipError_t launch_stream_gemm(const GemmArgs& p, int epi, int ops, int max_rows, int mblk, hipStream_t s);
 int gemm_out_cols_per_tile(int tile, int epi);
-// fp32 operands on the fp32 MFMA (v_mfma_f32_16x16x4f32): A, B and the output in fp32 (epi
-// kEpiSiluF32 or kEpiStoreF32); LDS-tiled kernels only (tiles 128x128, 32x128, 16x64).
+double expected_m_tiles(double rows, int bm);
+// fp32 operands: A, B and the output in fp32 (epi kEpiSiluF32 or kEpiStoreF32); LDS-tiled kernels only
+// (tiles 128x128, 64x128 and 32x128 on the bf16 MFMA over three bf16 terms per operand, 16x64 on the
+// fp32 MFMA v_mfma_f32_16x16x4f32).
 hipError_t launch_grouped_gemm_f32(const GemmArgs& p, int epi, int max_rows, int tile, hipStream_t s);
 
 // Base of expert e's weights: the pointer table when given, else b + e * b_estride elements.

@@ -220,7 +220,7 @@ def gemm_gate_up_silu(a: torch.Tensor, w_gate_up: torch.Tensor, seg_offsets: tor
                       a_rows: Optional[torch.Tensor] = None, w_scale: Optional[torch.Tensor] = None,
                       e_mod: Optional[int] = None, tile: int = 0) -> torch.Tensor:
     """fused_moe.py:445-459: h = silu(a.Wg^T) * (a.Wu^T) per segment -> bf16 [max_rows, I]
-    (fp32 a and weights: the fp32 MFMA, fp32 h)."""
+    (fp32 a and weights: fp32 h)."""
     f32 = w_gate_up.dtype == torch.float32
     _req(a, "a", torch.float32 if f32 else torch.bfloat16, 2)
     _req(w_gate_up, "w_gate_up", (torch.bfloat16, torch.float8_e4m3fn, torch.float32), 3)
@@ -250,7 +250,7 @@ def gemm_down(h: torch.Tensor, w_down: torch.Tensor, seg_offsets: torch.Tensor, 
               out_dtype=torch.float32, k_split: int = 1, w_scale: Optional[torch.Tensor] = None,
               e_mod: Optional[int] = None, tile: int = 0) -> torch.Tensor:
     """fused_moe.py:463-476: y = h . Wd^T per segment -> [k_split, max_rows, H] partial planes
-    (fp32 h and weights: the fp32 MFMA, fp32 y)."""
+    (fp32 h and weights: fp32 y)."""
     f32 = w_down.dtype == torch.float32
     _req(h, "h", torch.float32 if f32 else torch.bfloat16, 2)
     _req(w_down, "w_down", (torch.bfloat16, torch.float8_e4m3fn, torch.float32), 3)
@@ -360,7 +360,7 @@ def grouped_gemm(a: torch.Tensor, b: torch.Tensor, seg_offsets: torch.Tensor, ma
                  out_dtype=torch.bfloat16, a_rows: Optional[torch.Tensor] = None,
                  b_scale: Optional[torch.Tensor] = None, e_mod: Optional[int] = None, tile: int = 0) -> torch.Tensor:
     """single_group_gemm_moe.py:76-91: c[rows_s] = a[rows_s] . b[s % e_mod]^T, b packed [E,N,K]
-    (fp32 a and b: the fp32 MFMA, fp32 c)."""
+    (fp32 a and b: fp32 c)."""
     f32 = b.dtype == torch.float32
     _req(a, "a", torch.float32 if f32 else torch.bfloat16, 2)
     _req(b, "b", (torch.bfloat16, torch.float8_e4m3fn, torch.float32), 3)
@@ -463,7 +463,7 @@ def fused_moe(hidden_states: torch.Tensor, router_logits: torch.Tensor, top_k: i
     ``w_scales=(s_gate_up [E,2I], s_down [E,H])`` marks fp8-e4m3 weights: bf16 activations on
     the bf16 MFMA (W8A16), or with ``w8a8=True`` activations quantised per token / per row
     and both GEMMs on the fp8 MFMA (W8A8).
-    fp32 hidden states with fp32 weights run the fp32 layer (fp32 MFMA, fp32 h and y: the
+    fp32 hidden states with fp32 weights run the fp32 layer (fp32 products, h and y: the
     reference's fp32 F.linear path, native_moe.py:56-103); fp32 hidden states with bf16 or fp8
     weights are refused rather than rounded.
     The per-assignment expert outputs are kept in fp32 and summed by the combine in fp32 with one

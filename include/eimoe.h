@@ -53,8 +53,8 @@ enum {
                             (h = hi + lo, ~16 significant bits instead of 8) and the down projection
                             runs once per term (twice its time); y is kept in fp32.  Not with W8A8. */
   EIMOE_FP32 = 32        /* fp32 layer: x, the weights (w_dtype EIMOE_F32, shared weights too), h
-                            and y in fp32 on the fp32 MFMA (the reference's fp32 F.linear path,
-                            native_moe.py:56-103).  Required with, and only with, fp32 weights;
+                            and y in fp32, products to fp32's error (the reference's fp32 F.linear
+                            path, native_moe.py:56-103).  Required with, and only with, fp32 weights;
                             size the workspace with it.  Not with W8A8 or H_SPLIT. */
 };
 
@@ -154,7 +154,7 @@ int eimoe_gather(const void* x, int dtype, int H, const int32_t* rows, const int
  * directly; every a_rows entry must be < a_nrows, reads beyond the buffer return 0).
  * w_gate_up: [E_w, 2I, H] bf16 or fp8 (rows [0,I) gate, [I,2I) up, fused_moe.py:91-101);
  * w_scale: fp8 only, [E_w, 2I] fp32 per-output-channel scales.  h: bf16 [max_rows, I].
- * w_dtype EIMOE_F32: a and w_gate_up fp32 on the fp32 MFMA, h fp32 [max_rows, I].
+ * w_dtype EIMOE_F32: a and w_gate_up fp32, h fp32 [max_rows, I].
  * H % 64 == 0, I % 32 == 0.  max_rows bounds seg_offsets[n_seg]. */
 int eimoe_gemm_gate_up_silu(const void* a, const int32_t* a_rows, int a_nrows, int lda, const void* w_gate_up, int w_dtype,
                             const float* w_scale, int H, int I, const int32_t* seg_offsets, int n_seg, int e_mod,
@@ -162,7 +162,7 @@ int eimoe_gemm_gate_up_silu(const void* a, const int32_t* a_rows, int a_nrows, i
 
 /* Grouped down GEMM: y[r,:] = h[r,:] . W_d[e]^T (fused_moe.py:463-476).
  * h: bf16 [max_rows, I]; w_down: [E_w, H, I] bf16 or fp8 (+ w_scale [E_w, H]); or h and w_down
- * fp32 with w_dtype EIMOE_F32 (the fp32 MFMA; y_dtype EIMOE_F32).
+ * fp32 with w_dtype EIMOE_F32 (y_dtype EIMOE_F32).
  * y: y_dtype (EIMOE_F32 / EIMOE_BF16) [k_split][max_rows, H]; with k_split > 1 each K-slice
  * writes its own partial plane (summed by eimoe_combine), I/k_split % 64 == 0. */
 int eimoe_gemm_down(const void* h, int I, const void* w_down, int w_dtype, const float* w_scale, int H,

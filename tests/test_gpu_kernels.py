@@ -1010,3 +1010,51 @@ def test_ring_lds_tiles_bit_identical_with_two_stage(dev, tile, bm, bn, mode):
     assert torch.equal(gu(rows), gu(bounds["gu"]))
     for ks in (1, 2):
         assert torch.equal(dn(rows, ks), dn(bounds[f"dn{ks}"], ks))
+
+
+# The fp32 tiles of 32 rows and more multiply three bf16 terms per operand on the bf16 MFMA; a tile whose
+# sums are not finite, or nonzero below 2^-64, is computed again on the fp32 MFMA.  Every tile, on the
+# two-stage kernel and on the ring (row bounds in both regimes), against float64: ordinary values,
+# infinities, NaN, zero rows and the largest finite values, and operands near the smallest normal.
+# Bound: K rounded additions of partial sums below the norm n of the products, of rms 2^-24 n sqrt(K/2)
+# when taken as independent, six times that; the products left out are below 2^-22 each.  (A missing
+# term, or one cut at the smallest bf16, is 2^-16 n, three times the bound.)
+@pytest.mark.parametrize("tile", [2, 3, 6])
+@pytest.mark.parametrize("counts", [[33, 0, 70, 1], [400, 129, 700, 260]])
+@pytest.mark.parametrize("values", ["ordinary", "special", "tiny"])
+def test_fp32_split_terms(dev, tile, counts, values):
+    g = torch.Generator().manual_seed(101 + tile)
+    E, N, K = len(counts), 256, 320
+    off, off_t = _segments(counts)
+    rows = int(off[-1])
+    a = torch.randn(rows, K, generator=g)
+    b = torch.randn(E, N, K, generator=g)
+    if values == "special":
+        a[3, 7] = float("inf")
+        a[5, 0] = float("nan")
+        a[20] = 0.0
+        a[21] = 3.4e38
+        b[2, 9, 11] = -float("inf")
+        b[2, 40, 3] = 3.4028234663852886e38
+    elif values == "tiny":
+        a *= 2.0 ** -118
+        b *= 2.0 ** 30
+    c = cpu(ops.grouped_gemm(a.to(dev), b.to(dev), off_t.to(dev), rows, out_dtype=torch.float32, tile=tile))
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        x, w = a[lo:hi].double(), b[e].double()
+        ref = x @ w.T
+        got = c[lo:hi].double()
+        fin = torch.isfinite(ref) & (ref.abs() < 3.4e38)
+        if values == "special":
+            # a sum past fp32 in the middle of a row may end infinite or NaN: only rows and columns
+            # without the largest values are compared value by value
+            plain = (x.abs().amax(1) < 1e30)[:, None] & (w.abs().amax(1) < 1e30)[None, :]
+            special = ~torch.isfinite(x).all(1)[:, None] | ~torch.isfinite(w).all(1)[None, :]
+            assert torch.equal(torch.isnan(got)[special], torch.isnan(ref)[special])
+            assert torch.equal(got[special & torch.isinf(ref)], ref[special & torch.isinf(ref)])
+            assert not torch.isfinite(got[~(ref.abs() <= 3.4029e38)]).any()   # past the largest fp32
+            fin &= plain
+        norm = ((x[:, None, :] * w[None, :, :]) ** 2).sum(-1).sqrt()
+        err = (got - ref).abs()
+        assert (err[fin] <= 6 * math.sqrt(K / 2) * 2.0 ** -24 * norm[fin]).all()
