@@ -149,7 +149,7 @@ hipError_t launch_router_topk(const float* logits, int T, int E, int k, int reno
 // softmax router compare logits), so s is computed in double and rounded once to fp32:
 // the correctly rounded sigmoid, which the oracle computes the same way.  Ties go to the
 // lower group / expert id; the picks come out in descending order of c.
-// One wave per token (kGroupedWaves per workgroup); lane l holds experts l*VPL..+VPL-1.
+// General form: one wave per token (kGroupedWaves per workgroup); lane l holds experts l*VPL..+VPL-1.
 // Group scores and group selection go through LDS, so any n_group dividing E works.
 constexpr int kGroupedWaves = 4;
 constexpr int kGroupedMaxE = 512;
@@ -285,11 +285,190 @@ __global__ __launch_bounds__(64 * kGroupedWaves) void router_grouped_kernel(
   }
 }
 
+// The same gate with a token per 16-lane DPP row: lane l of a row holds experts l*VPL..+VPL-1 of E =
+// 16*VPL, a group is gsize/VPL neighbouring lanes (a power of two), and the reductions (top 2 of a group,
+// the k argmax rounds) are VALU lane permutes within the row, where the wave-wide form spends ~200
+// dependent LDS-routed shuffles.  TPW tokens per wave: 4, a row each, or 1 (small batches), whose sigmoids
+// then take the whole wave and whose rows all select the same picks.  Latency-bound: the sigmoids (double
+// precision, four at a time in a rolled loop; unrolled they were a chain of 16 and 10 KiB of code), then
+// k rounds over keys that order as the scores do.  DeepSeek-V3 gate (256 experts, 8 groups, top 8), 4096
+// tokens 27.0 -> 8.5 us; 777 tokens over 64 experts, top 6, 10.1 -> 6.4 us.  Same comparisons on the same values, sums in the same order: bit-identical.
+template <int VPL, int TPW>
+__global__ __launch_bounds__(64 * kGroupedWaves) void router_grouped_row_kernel(
+    const float* __restrict__ logits, int T, int k, int n_group, int topk_group, const float* __restrict__ bias,
+    int renorm, float scaling, int32_t* __restrict__ ids, float* __restrict__ wts) {
+  constexpr int E = 16 * VPL;
+  constexpr int LP = 64 / TPW;   // lanes per token in the sigmoid phase
+  __shared__ __attribute__((aligned(16))) float s_sg[kGroupedWaves * TPW][E];
+  const int lane = threadIdx.x & 63;
+  const int wv = threadIdx.x >> 6;
+  const int li = lane & 15;
+  const int row0 = lane & 48;   // the row's first lane
+  const int slot = TPW == 1 ? wv : wv * 4 + (lane >> 4);
+  const int t = blockIdx.x * (kGroupedWaves * TPW) + slot;
+  const bool tv = t < T;
+  const float NEG_INF = -__builtin_inff();
+  const int lg = 16 / n_group;   // lanes per group
+
+  float c[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) c[j] = 0.f;
+  if (bias) {
+#pragma unroll
+    for (int q = 0; q < VPL; q += 4) {
+      const float4 v = *reinterpret_cast<const float4*>(bias + li * VPL + q);
+      c[q] = v.x;
+      c[q + 1] = v.y;
+      c[q + 2] = v.z;
+      c[q + 3] = v.w;
+    }
+  }
+  float4* sg4 = reinterpret_cast<float4*>(s_sg[slot]);
+  const int l0 = lane % LP;
+  {
+    const float4* src = reinterpret_cast<const float4*>(logits + static_cast<long long>(tv ? t : T - 1) * E);
+    float4 v[(E / 4 + LP - 1) / LP];
+#pragma unroll
+    for (int q = 0; q < E / 4; q += LP)
+      if (q + LP <= E / 4 || q + l0 < E / 4) v[q / LP] = src[q + l0];
+#pragma unroll
+    for (int q = 0; q < E / 4; q += LP)
+      if (q + LP <= E / 4 || q + l0 < E / 4) sg4[q + l0] = v[q / LP];
+  }
+#pragma unroll 1
+  for (int q = l0; q < E / 4; q += LP) {   // each lane its own vectors
+    float4 v = sg4[q];
+    v.x = sigmoid_rn(v.x);
+    v.y = sigmoid_rn(v.y);
+    v.z = sigmoid_rn(v.z);
+    v.w = sigmoid_rn(v.w);
+    sg4[q] = v;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  float a1 = NEG_INF, a2 = NEG_INF;
+#pragma unroll
+  for (int q = 0; q < VPL; q += 4) {
+    const float4 v = sg4[(li * VPL + q) / 4];
+    c[q] = v.x + c[q];
+    c[q + 1] = v.y + c[q + 1];
+    c[q + 2] = v.z + c[q + 2];
+    c[q + 3] = v.w + c[q + 3];
+  }
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {   // a NaN counts for nothing
+    const float v = c[j] == c[j] ? c[j] : NEG_INF;
+    a2 = fmaxf(a2, fminf(a1, v));
+    a1 = fmaxf(a1, v);
+  }
+  // group scores: the top 2 over the group's lanes, in every one of them
+  auto merge = [&](float b1, float b2) {
+    const float hi = fmaxf(a1, b1);
+    a2 = fmaxf(fminf(a1, b1), fmaxf(a2, b2));
+    a1 = hi;
+  };
+  if (lg >= 2) merge(dpp_f<0xB1>(a1), dpp_f<0xB1>(a2));     // quad_perm [1,0,3,2]
+  if (lg >= 4) merge(dpp_f<0x4E>(a1), dpp_f<0x4E>(a2));     // quad_perm [2,3,0,1]
+  if (lg >= 8) merge(dpp_f<0x141>(a1), dpp_f<0x141>(a2));   // row_half_mirror
+  if (lg >= 16) merge(dpp_f<0x140>(a1), dpp_f<0x140>(a2));  // row_mirror
+  // keep the topk_group best groups (ties to the lower group index)
+  const float score = a1 + a2;
+  const int g = li / lg;
+  int rank = 0;
+  for (int h = 0; h < n_group; ++h) {
+    const float u = __shfl(score, row0 + h * lg, 64);
+    rank += ((u > score) | ((u == score) & (h < g))) ? 1 : 0;
+  }
+  // Keys that order as the masked scores do (-0 as +0): 0 is below every score, for NaN and for what has
+  // been picked.
+  const bool kept = rank < topk_group;
+  uint32_t key[VPL];
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const float v = kept ? c[j] + 0.f : 0.f;
+    const uint32_t u = __float_as_uint(v);
+    const uint32_t o = u ^ (static_cast<uint32_t>(static_cast<int32_t>(u) >> 31) | 0x80000000u);
+    key[j] = v == v ? o : 0u;
+  }
+  // top-k of the masked scores; pick r is kept by lane r % 16 of the row (k <= 32)
+  int my_id0 = -1, my_id1 = -1;
+#pragma unroll 1
+  for (int r = 0; r < k; ++r) {
+    uint32_t bv = 0u;
+    int bi = 0x7fffffff;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {   // ascending ids: a tie keeps the lower one
+      const bool better = key[j] > bv;
+      bv = better ? key[j] : bv;
+      bi = better ? li * VPL + j : bi;
+    }
+    auto take = [&](uint32_t ov, int oi) {
+      const bool better = (ov > bv) | ((ov == bv) & (oi < bi));
+      bv = better ? ov : bv;
+      bi = better ? oi : bi;
+    };
+    take(dpp_i<0xB1>(bv), dpp_i<0xB1>(bi));
+    take(dpp_i<0x4E>(bv), dpp_i<0x4E>(bi));
+    take(dpp_i<0x141>(bv), dpp_i<0x141>(bi));
+    take(dpp_i<0x140>(bv), dpp_i<0x140>(bi));
+    my_id0 = r == li ? bi : my_id0;
+    my_id1 = r == li + 16 ? bi : my_id1;
+    const int mine = bi - li * VPL;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) key[j] = mine == j ? 0u : key[j];
+  }
+  // weight = unbiased sigmoid of the pick (a row short of scores has picks without one: the last expert's)
+  float w0 = li < k ? s_sg[slot][min(my_id0, E - 1)] : 0.f;
+  float w1 = li + 16 < k ? s_sg[slot][min(my_id1, E - 1)] : 0.f;
+  if (renorm && k > 1) {
+    float sum = w0 + w1;
+#pragma unroll
+    for (int m = 8; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, 64);
+    w0 = w0 / (sum + 1e-20f);
+    w1 = w1 / (sum + 1e-20f);
+  }
+  if (!tv || (TPW == 1 && lane >= 16)) return;
+  if (li < k) {
+    ids[static_cast<long long>(t) * k + li] = my_id0;
+    wts[static_cast<long long>(t) * k + li] = w0 * scaling;
+  }
+  if (li + 16 < k) {
+    ids[static_cast<long long>(t) * k + li + 16] = my_id1;
+    wts[static_cast<long long>(t) * k + li + 16] = w1 * scaling;
+  }
+}
+
 hipError_t launch_router_grouped(const float* logits, int T, int E, int k, int n_group, int topk_group,
                                  const float* bias, int renorm, float scaling, int32_t* ids, float* w,
                                  hipStream_t s) {
+  const dim3 b(64 * kGroupedWaves);
+  // A token per 16-lane row where the row's lanes hold whole 16-byte vectors and a group is a power of two
+  // of lanes; the wave-wide kernel for the other expert and group counts and for unaligned arrays.  One
+  // token per wave while that leaves at most one wave per SIMD.
+  if (T > 0 && (E == 64 || E == 128 || E == 256) && n_group <= 16 && 16 % n_group == 0 &&
+      (reinterpret_cast<uintptr_t>(logits) | reinterpret_cast<uintptr_t>(bias)) % 16 == 0) {
+    const int tpw = T <= 4 * kNumCu ? 1 : 4;
+    const dim3 g(static_cast<unsigned>((T + tpw * kGroupedWaves - 1) / (tpw * kGroupedWaves)));
+#define EIMOE_RGR(V, N)                                                                                            \
+  hipLaunchKernelGGL((router_grouped_row_kernel<V, N>), g, b, 0, s, logits, T, k, n_group, topk_group, bias, renorm, \
+                     scaling, ids, w)
+#define EIMOE_RGR_T(V) \
+  if (tpw == 1) EIMOE_RGR(V, 1); \
+  else EIMOE_RGR(V, 4)
+    if (E == 64) {
+      EIMOE_RGR_T(4);
+    } else if (E == 128) {
+      EIMOE_RGR_T(8);
+    } else {
+      EIMOE_RGR_T(16);
+    }
+#undef EIMOE_RGR_T
+#undef EIMOE_RGR
+    return hipGetLastError();
+  }
   const unsigned blocks = static_cast<unsigned>((T + kGroupedWaves - 1) / kGroupedWaves);
-  const dim3 g(blocks > 0 ? blocks : 1), b(64 * kGroupedWaves);
+  const dim3 g(blocks > 0 ? blocks : 1);
   const int vpl = (E + 63) / 64;
 #define EIMOE_RG(V) \
   hipLaunchKernelGGL((router_grouped_kernel<V>), g, b, 0, s, logits, T, E, k, n_group, topk_group, bias, renorm, \

@@ -87,6 +87,32 @@ def test_router_grouped_ties_and_masked_zeros(dev):
         torch.testing.assert_close(cpu(w), rw, rtol=2e-6, atol=1e-7)
 
 
+# The token-per-row kernel (64, 128 or 256 experts in up to 16 groups, a power of two, 16-byte aligned
+# logits) against the wave-wide one, which takes the same logits off alignment: bit for bit, with ties,
+# infinities and NaN, ragged token counts, every group count and both pick slots.
+@pytest.mark.parametrize("E", [64, 128, 256])
+@pytest.mark.parametrize("ng", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("T,k,norm,use_bias", [(1, 1, True, True), (67, 16, False, False), (1024, 8, True, True),
+                                               (1027, 32, True, True)])
+def test_router_grouped_row_kernel_bit_identical(dev, E, ng, T, k, norm, use_bias):
+    g = torch.Generator().manual_seed(E + ng + T)
+    logits = torch.randn(T, E, generator=g) * 2.0
+    logits[T // 2] = torch.randint(-2, 3, (E,), generator=g).float()
+    logits[T - 1, ::7] = float("inf")
+    logits[0, 1::5] = -float("inf")
+    if T > 3:
+        logits[2, ::3] = float("nan")
+        logits[3] = float("nan")
+    bias = (torch.randn(E, generator=g) * 0.1).to(dev) if use_bias else None
+    buf = torch.empty(T * E + 1, device=dev)
+    buf[1:] = logits.reshape(-1).to(dev)
+    tg = max(1, ng // 2)
+    ids0, w0 = ops.router_grouped_topk(buf[1:].view(T, E), k, ng, tg, bias, norm, 2.5)
+    ids1, w1 = ops.router_grouped_topk(logits.to(dev), k, ng, tg, bias, norm, 2.5)
+    assert torch.equal(cpu(ids0), cpu(ids1))
+    assert torch.equal(cpu(w0).view(torch.int32), cpu(w1).view(torch.int32))
+
+
 def test_router_grouped_empty(dev):
     ids, w = ops.router_grouped_topk(torch.empty(0, 64, device=dev), 6, 8, 4)
     assert ids.shape == (0, 6)
