@@ -588,12 +588,19 @@ int eimoe_gemm_down_w8a8(const void* hq, const float* h_scale, int I, const void
 
 namespace {
 
+// Blocks (source rank, weight) to be regrouped by weight before the GEMM: the maps it then reads.
+struct BlockMerge {
+  const int32_t* counts;
+  int n_seg;
+  int32_t *offsets, *rows, *pos;
+};
+
 // The grouped GEMM of the op point, expert weights either packed (b, b_expert_stride elements
 // apart) or one [N, K] matrix per expert through a device table of b_ptrs.
 int grouped_gemm_impl(const void* a, const int32_t* a_rows, int a_nrows, int lda, const void* b,
                       const void* const* b_ptrs, int b_dtype, const float* b_scale, long long b_expert_stride, int N,
                       int K, const int32_t* seg_offsets, int n_seg, int e_mod, int max_rows, void* c, int c_dtype,
-                      int tile, void* stream) {
+                      int tile, void* stream, const BlockMerge* merge = nullptr) {
   int rc = check_gemm_common(max_rows, n_seg, e_mod);
   if (rc) return rc;
   if (b_dtype != EIMOE_BF16 && b_dtype != EIMOE_FP8 && b_dtype != EIMOE_F32)
@@ -618,6 +625,10 @@ int grouped_gemm_impl(const void* a, const int32_t* a_rows, int a_nrows, int lda
   REQUIRE_PTR(seg_offsets);
   REQUIRE_PTR(c);
   if (b_dtype == EIMOE_FP8) REQUIRE_PTR(b_scale);
+  if (merge && (rc = hip_check(launch_merge_segments(merge->counts, merge->n_seg, n_seg, max_rows, merge->offsets,
+                                                     merge->rows, merge->pos, S(stream)),
+                               "merge segments")))
+    return rc;
   GemmArgs p{};
   p.a = a;
   p.a_rows = a_rows;
@@ -634,6 +645,7 @@ int grouped_gemm_impl(const void* a, const int32_t* a_rows, int a_nrows, int lda
   p.S = n_seg;
   p.e_mod = e_mod;
   p.c = c;
+  p.c_rows = merge ? merge->rows : nullptr;
   p.ldc = N;
   p.k_split = 1;
   p.max_rows = max_rows;
@@ -662,6 +674,33 @@ int eimoe_grouped_gemm_ptrs(const void* a, const int32_t* a_rows, int a_nrows, i
   return grouped_gemm_impl(a, a_rows, a_nrows, lda, nullptr, b_ptrs, EIMOE_BF16, nullptr,
                            static_cast<long long>(N) * K, N, K, seg_offsets, n_seg, e_mod, max_rows, c, c_dtype, tile,
                            stream);
+}
+
+size_t eimoe_grouped_gemm_blocks_workspace_bytes(int M, int n_b) {
+  if (M < 0 || n_b < 1) return 0;
+  return align256(static_cast<size_t>(n_b + 1) * 4) + 2 * align256(static_cast<size_t>(M) * 4);
+}
+
+int eimoe_grouped_gemm_blocks(const void* a, int M, int lda, const void* const* b_ptrs, int n_b, int N, int K,
+                              const int32_t* counts, int n_seg, void* c, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+  int rc = check_gemm_common(M, n_seg, n_b);
+  if (rc) return rc;
+  if (n_seg % n_b) return fail(EIMOE_ERR_SHAPE, "n_seg=%d not a multiple of n_b=%d", n_seg, n_b);
+  if (M == 0)
+    return grouped_gemm_impl(a, nullptr, M, lda, nullptr, b_ptrs, EIMOE_BF16, nullptr, static_cast<long long>(N) * K,
+                             N, K, nullptr, n_b, n_b, M, c, EIMOE_BF16, EIMOE_TILE_AUTO, stream);
+  REQUIRE_PTR(counts);
+  REQUIRE_PTR(b_ptrs);
+  REQUIRE_PTR(workspace);
+  const size_t need = eimoe_grouped_gemm_blocks_workspace_bytes(M, n_b);
+  if (workspace_bytes < need)
+    return fail(EIMOE_ERR_WORKSPACE, "workspace %zu bytes < required %zu", workspace_bytes, need);
+  BlockMerge m{counts, n_seg, static_cast<int32_t*>(workspace), nullptr, nullptr};
+  m.rows = m.offsets + align256(static_cast<size_t>(n_b + 1) * 4) / 4;
+  m.pos = m.rows + align256(static_cast<size_t>(M) * 4) / 4;
+  return grouped_gemm_impl(a, m.rows, M, lda, nullptr, b_ptrs, EIMOE_BF16, nullptr, static_cast<long long>(N) * K, N, K,
+                           m.offsets, n_b, n_b, M, c, EIMOE_BF16, EIMOE_TILE_AUTO, stream, &m);
 }
 
 int eimoe_combine(const void* y, int y_dtype, int n_split, long long split_stride, const int32_t* pos,

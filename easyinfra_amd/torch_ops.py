@@ -9,7 +9,8 @@ contiguous blocks, ``B_list`` one ``[N,K]`` nn.Linear weight per block,
 grouped GEMM.  The weights are read where they lie, through a device table of
 per-expert pointers: the reference's list holds its experts' Parameters repeated
 ep_size times (single_group_gemm_moe.py:73-76, 89), so only the first period goes
-into the table and the blocks index it modulo its length.  No weight is copied.
+into the table and the blocks index it modulo its length.  Blocks of one weight are computed as
+one segment.  No weight is copied.
 """
 from __future__ import annotations
 
@@ -32,8 +33,8 @@ def _period(b_list: List[torch.Tensor]) -> int:
     """Shortest p with b_list[i] the same tensor memory as b_list[i % p] for every i."""
     n = len(b_list)
     ptrs = [b.data_ptr() for b in b_list]
-    for p in range(1, n + 1):
-        if n % p == 0 and all(ptrs[i] == ptrs[i % p] for i in range(n)):
+    for p in range(1, n):
+        if n % p == 0 and ptrs[p:] == ptrs[:-p]:
             return p
     return n
 
@@ -71,19 +72,28 @@ def hip_grouped_gemm_single(A: torch.Tensor, B_list: List[torch.Tensor], block_s
     A = A.contiguous()
     ops._req(A, "A", torch.bfloat16, 2)
     N, K = B_list[0].shape
+    p = _period(B_list)
     for i, b in enumerate(B_list):
+        if i >= p and b is B_list[i - p]:   # checked already
+            continue
         ops._req(b, f"B_list[{i}]", torch.bfloat16, 2)
         if tuple(b.shape) != (N, K) or b.device != A.device:
             raise ValueError(f"B_list[{i}] is {tuple(b.shape)} on {b.device}, expected ({N}, {K}) on {A.device}")
     if K != A.shape[1]:
         raise ValueError(f"A has {A.shape[1]} columns, the weights K={K}")
-    p = _period(B_list)
     table = _ptr_table(B_list[:p], A.device)
+    c = torch.empty(M, N, dtype=A.dtype, device=A.device)
+    if p < len(block_sizes):
+        counts = _to_device([int(b) for b in block_sizes], torch.int32, A.device)
+        need = int(_lib.lib().eimoe_grouped_gemm_blocks_workspace_bytes(M, p))
+        ws = torch.empty(need, dtype=torch.uint8, device=A.device)
+        call("eimoe_grouped_gemm_blocks", A.data_ptr(), M, A.stride(0), table.data_ptr(), p, N, K, counts.data_ptr(),
+             len(block_sizes), c.data_ptr(), ws.data_ptr(), need, ops._stream(A))
+        return c
     bounds = [0]
     for b in block_sizes:
         bounds.append(bounds[-1] + int(b))
     off = _to_device(bounds, torch.int32, A.device)
-    c = torch.empty(M, N, dtype=A.dtype, device=A.device)
     call("eimoe_grouped_gemm_ptrs", A.data_ptr(), None, A.shape[0], A.stride(0), table.data_ptr(), p, N, K,
          off.data_ptr(), len(block_sizes), p, M, c.data_ptr(), _lib.BF16, 0, ops._stream(A))
     return c

@@ -214,6 +214,16 @@ int eimoe_grouped_gemm_ptrs(const void* a, const int32_t* a_rows, int a_nrows, i
                             int n_b, int N, int K, const int32_t* seg_offsets, int n_seg, int e_mod, int max_rows,
                             void* c, int c_dtype, int tile, void* stream);
 
+/* The op point's grouped GEMM where its list repeats the same n_b weights once per source rank: block
+ * s of A holds counts[s] rows (device int32, n_seg a multiple of n_b) and multiplies b_ptrs[s % n_b];
+ * c [M, N] bf16 keeps A's row order.  Blocks of one weight are computed as one segment, so a weight is
+ * read once however many ranks sent rows.  Same operands and limits as eimoe_grouped_gemm_ptrs;
+ * workspace: eimoe_grouped_gemm_blocks_workspace_bytes bytes. */
+size_t eimoe_grouped_gemm_blocks_workspace_bytes(int M, int n_b);
+int eimoe_grouped_gemm_blocks(const void* a, int M, int lda, const void* const* b_ptrs, int n_b, int N, int K,
+                              const int32_t* counts, int n_seg, void* c, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
 /* Weighted top-k combine: out[t,:] = sum_j w[t,j] * sum_s y[s][pos[t*k+j],:]  (+ shared_y[t,:]).
  * Replaces _all2all_chunk_output_compute (blocks/moe/moe_all2all.py:291-307) and the shared-expert
  * residual add (moe_all2all.py:535-537).  Slots with pos < 0 contribute nothing; a token with no

@@ -72,3 +72,35 @@ def test_experts_match_oracle_per_segment(dev, E, ep, H, I, pattern, mode):
     # flips with the order of the fp32 sums (far fewer); W8A16 forms the oracle's products with the
     # scale applied to the sum instead of the weight (fp32 rounding).  fp32: sums of up to 16384 terms.
     assert oracle.rel_l2(y.cpu().float(), ref) <= (2e-5 if mode == "fp32" else 2.0 ** -8)
+
+
+def test_grouped_gemm_blocks_validation():
+    f = _lib.lib().eimoe_grouped_gemm_blocks
+    ok = dict(a=1, M=8, lda=128, b=1, n_b=4, N=128, K=128, c=1, S=8, out=1, ws=1, wsb=1 << 30, st=None)
+    rc = lambda **kw: f(*dict(ok, **kw).values())
+    assert rc(S=6) == _lib.ERR_SHAPE                      # blocks not a multiple of the weights
+    assert rc(S=2000, n_b=2) == _lib.ERR_SHAPE and rc(lda=64) == _lib.ERR_SHAPE
+    assert rc(K=100) == _lib.ERR_ALIGN and rc(N=96) == _lib.ERR_ALIGN
+    assert rc(c=None) == _lib.ERR_NULL and rc(a=None) == _lib.ERR_NULL
+    assert rc(wsb=16) == _lib.ERR_WORKSPACE
+    assert rc(M=1 << 23) == _lib.ERR_SHAPE                # A: 2 GiB
+    assert rc(M=0, a=None) == _lib.EIMOE_OK
+
+
+# The op point on lists that repeat their weights (blocks of one weight multiplied as one segment) against
+# the oracle per block.
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,ep,K,N,pattern", [(4, 2, 128, 192, "one"), (5, 3, 192, 128, "edges"), (3, 4, 256, 256, "hot"),
+                                              (1, 8, 128, 128, "edges"), (65, 2, 64, 64, "few"),
+                                              (2, 3, 4096, 4096, "edges")])
+def test_op_point_merges_repeated_weights(dev, E, ep, K, N, pattern):
+    import easyinfra_amd.torch_ops  # noqa: F401
+    g = torch.Generator().manual_seed(E * ep + N)
+    blocks = [int(v) for v in _counts(E, ep, pattern, E).reshape(-1)]
+    a = torch.randn(sum(blocks), K, generator=g).to(torch.bfloat16)
+    w = [(torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16) for _ in range(E)]
+    print("CASE", dict(E=E, ep=ep, K=K, N=N, pattern=pattern), flush=True)
+    out = torch.ops.ops.hip_grouped_gemm_single(a.to(dev), [b.to(dev) for b in w] * ep, blocks)
+    ref = oracle.grouped_gemm(a, w * ep, blocks)
+    # one bf16 rounding of the output, at most 2^-9 of each value; fp32 sums of up to 4096 terms
+    assert oracle.rel_l2(out.cpu().float(), ref) <= 2.0 ** -8
