@@ -111,7 +111,10 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
   q.nb_rows = H;
   // the tile the launch will take (the W8A16 layer is costed as bf16: its workspace query does not
   // see the weight type; any split chosen here is valid for it, at worst on its LDS tiles)
-  const int tile = gemm_choose_tile(q, kEpiStoreF32, w8a8, w8a8);
+  int tile = gemm_choose_tile(q, kEpiStoreF32, w8a8, w8a8);
+  if (!w8a8 && tile != kTileStream && few_large_down(n_local, H, static_cast<double>(H) * I * 2))
+    tile = few_large_down_tile(n_local, static_cast<double>(rows_hint > 0 ? std::min(rows_hint, max_rows) : max_rows) /
+                                            n_local);
   if (tile == kTileStream) {
     // Few rows per segment: the weight-streaming kernel runs one workgroup per (segment,
     // column group, 32-row chunk, split).  Split until there are about 6 workgroups per CU
@@ -130,18 +133,28 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
   // best (Mixtral 64 tokens, 128x128 bf16: split 1/2/4/8 = 226/159/163/171 us; 32x128
   // e4m3: 109/84/99/94).
   const double expert_bytes = static_cast<double>(H) * I * (w8a8 ? 1 : 2);
-  if (expert_bytes >= 32.0 * 1024 * 1024 && tile != kTileL)
-    return (I / (w8a8 ? 128 : 64)) % 2 == 0 ? 2 : 1;
-  if (w8a8) I /= 2;   // e4m3 tiles run at twice the bf16 rate: cost them as half the K
   const int bm = tile == kTileL ? 256 : tile == kTileM ? 128 : tile == kTileMS ? 64 : tile == kTileS ? 32 : 16;
   const int bn = gemm_out_cols_per_tile(tile, kEpiStoreF32);
   const int rows = rows_hint > 0 ? std::min(rows_hint, max_rows) : max_rows;
-  // m-tiles in full-tile units from the expected rows per segment: whole tiles plus the remainder's
-  // tile, which takes a quarter, half or full height (a short tile costs its share of a round)
   const int segs = std::max(1, std::min(n_local, rows));
   const double per = static_cast<double>(rows) / segs;
+  if (expert_bytes >= 32.0 * 1024 * 1024 && tile != kTileL) {
+    const int steps = I / (w8a8 ? 128 : 64);
+    if (steps % 2) return 1;
+    // one or two experts: split until there is a workgroup per CU (figures at few_large_down)
+    const long long wgs = static_cast<long long>(segs * std::ceil(per / bm)) * (H / bn);
+    int split = 2;
+    while (split < 8 && wgs * split * 2 <= kNumCu && steps % (split * 2) == 0) split *= 2;
+    return split;
+  }
+  if (w8a8) I /= 2;   // e4m3 tiles run at twice the bf16 rate: cost them as half the K
+  // m-tiles in full-tile units from the expected rows per segment: whole tiles plus the remainder's
+  // tile, which takes a quarter, half or full height (a short tile costs its share of a round)
+  const bool one_seg = n_local == 1 && rows_hint <= 0;   // an expert whose rows are known
   double mt;
-  if (tile == kTileL) {
+  if (one_seg) {
+    mt = std::ceil(per / bm);
+  } else if (tile == kTileL) {
     // The persistent 256x256 kernel: every m-tile of a segment costs about a full tile whatever its
     // height, and routed segments scatter around the mean, so an expected count just past a
     // multiple of 256 rows gives about half the segments one more m-tile.  Count
@@ -156,7 +169,9 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
   }
   const double work = mt * (H / bn);                                              // full-tile units
   const long long tiles = static_cast<long long>(segs * std::ceil(per / bm)) * (H / bn);   // workgroups
-  constexpr double kTileFlops = 4.7e12;   // measured bf16 GEMM rate per CU, FLOP/s
+  // measured bf16 GEMM rate per CU, FLOP/s; the launches of one expert end before the chip's power
+  // limit lowers the clock (Mixtral-8x7B down, one round of 256x256 tiles: 258 us at 3000 rows)
+  const double kTileFlops = one_seg ? 7.0e12 : 4.7e12;
   constexpr double kHbm = 5.0e12;         // achieved HBM rate for plane traffic, B/s
   const double t_tile = 2.0 * bm * bn * static_cast<double>(I) / kTileFlops;
   const double t_plane = 2.0 * static_cast<double>(max_rows) * H * y_elem / kHbm;
@@ -173,7 +188,8 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
     double cost = rounds / split * t_tile + (split - 1) * t_plane;
     // too few workgroups to fill the GPU: twice over for the one-tile-per-workgroup kernels, once
     // for the persistent 256x256 one (whose workgroups walk their tiles)
-    const bool few = tile == kTileL ? work * split < kNumCu : items < 2 * kNumCu;
+    // (one expert: three quarters, 1500 Mixtral-8x7B rows 177 us with 4 splits, 148 with 2)
+    const bool few = tile == kTileL ? work * split < (one_seg ? 0.75 : 1.0) * kNumCu : items < 2 * kNumCu;
     if (few && split < 8 && I % (128 * split) == 0) cost = 1e300;
     if (cost < best_cost * 0.98) {
       best_cost = cost;

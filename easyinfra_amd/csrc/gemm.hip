@@ -2282,25 +2282,63 @@ int gemm_out_cols_per_tile(int tile, int epi) {
 //    174.3 / 178.6 / 218.9 on 64x128 / 128x128 / 32x128, down 88.2 against 99.5 / 105.1 / 115.3
 //    (uniform routing: 168.7 and 87.2 on 256x256); 128 tokens (12 rows): gate/up 112.6 on 128x128
 //    against 125.3 streamed and 128.4 on 32x128.
+// bf16 since the 64x128 tile runs on the ring, on segments an eighth of which hold 8 times the rows of the
+// others (cold, one box; us; expected rows per segment in brackets): gate/up, Qwen3 share 512 / 2048 / 4100
+// rows [16 / 64 / 128] 40.9 / 55.6 / 61.7 on 64x128, 48.8 / 52.2 / 75.7 on 128x128, 46.4 / 44.6 / 46.3 on
+// 256x256 (one round of 240 tiles); 16 DeepSeek-V2-Lite experts 256 / 1024 / 2048 rows [16 / 64 / 128] 37.5 /
+// 54.9 / 70.5, 45.9 / 50.2 / 73.0 and 43.9 / 41.7 / 44.1.  A 256x256 tile takes about the same time whatever
+// its height, so it wins once the rows would need a second round of the small tiles, down to half a
+// round of tiles.
 static int routed_small_gate_up_tile(const GemmArgs& p, int S, double avg, int t, bool fp8) {
   const long long tiles_l = static_cast<long long>(S) * static_cast<long long>((avg + 255) / 256) * (p.N / 128);
-  const long long tiles_m = static_cast<long long>(S) * static_cast<long long>((avg + 127) / 128) * (p.N / 64);
   const long long tiles_ms = static_cast<long long>(S) * static_cast<long long>((avg + 63) / 64) * (p.N / 64);
+  const long long tiles_m = static_cast<long long>(S) * static_cast<long long>((avg + 127) / 128) * (p.N / 64);
+  if (!fp8) {
+    if (avg >= 40 && tiles_l >= kNumCu / 2) return kTileL;
+    return avg >= (tiles_m >= 2 * kNumCu ? 8 : 16) && avg < 64 ? kTileMS : t;
+  }
   if (avg >= 40 && tiles_l >= kNumCu) return kTileL;
-  if (avg >= 20 && avg < 64 && (!fp8 || tiles_ms <= 3 * kNumCu)) return kTileMS;
+  if (avg >= 20 && avg < 64 && tiles_ms <= 3 * kNumCu) return kTileMS;
   if (avg >= 8 && avg < 20 && tiles_m >= 2 * kNumCu) return kTileM;
   return t;
 }
 
 // e4m3 (W8A8) tiles do half the MFMA work per weight byte: the 64x128 band reaches to 80 rows, the
 // 256x256 tile takes over from 64, and below 40 rows the 32x128 tile (t) stays.
+// bf16 (as above, us on 64x128 / 128x128 / 256x256): down, Qwen3 share 1024 / 2048 / 8192 rows [32 / 64 / 256]
+// 24.2 / 35.8 / 23.9, 28.3 / 34.5 / 36.0 and 51.5 / 56.6 / 45.6; 32 DeepSeek-V2-Lite experts 2048 / 8192 rows
+// [64 / 256] 43.6 / 55.0 / 54.7 and 97.4 / 85.3 / 69.4; the op point (N 1536, K 2048) 512 / 2048 / 4100 rows
+// [16 / 64 / 128] 36.4 / 43.3 / 41.0, 56.1 / 45.7 / 41.6 and 66.3 / 76.0 / 44.9, over 64 weights (N 2816) 2048
+// rows [32] 137.7 / 182.0 / 134.9.  256x256 where its tiles, a quarter more than segments for the skew, make
+// one round or from two rounds on; between them its second round is nearly empty.
 static int routed_small_down_tile(const GemmArgs& p, int S, double avg, int t, bool fp8) {
   const long long tiles_ms = static_cast<long long>(S) * static_cast<long long>((avg + 63) / 64) * (p.N / 128);
   const long long tiles_l = static_cast<long long>(S) * static_cast<long long>((avg + 255) / 256) * (p.N / 256);
-  if (avg >= 20 && avg < (fp8 ? 80 : 64) && tiles_ms <= 3 * kNumCu) return kTileMS;   // one round of 64x128 workgroups
-  if (avg >= (fp8 ? 64 : 36) && tiles_l >= 2 * kNumCu) return kTileL;
-  if (fp8 && avg < 40) return t;
-  return kTileM;
+  if (!fp8) {
+    // (below 12 rows the two are level, 18.4 each at 4 rows and 21.2 at 8, unless 128x128 makes no more tiles than
+    // CUs: 16 experts, 128 rows 23.9 -> 17.9 us; the Qwen3 share's layer at 128 tokens is 2 us slower on 64x128)
+    if (avg < 40) return avg >= 12 || static_cast<long long>(S) * (p.N / 128) <= kNumCu ? kTileMS : kTileM;
+    if ((tiles_l >= kNumCu / 2 && tiles_l * 5 <= kNumCu * 4) || tiles_l >= 2 * kNumCu || avg >= 200) return kTileL;
+    return avg < 72 ? kTileMS : kTileM;
+  }
+  if (avg >= 20 && avg < 80 && tiles_ms <= 3 * kNumCu) return kTileMS;   // one round of 64x128 workgroups
+  if (avg >= 64 && tiles_l >= 2 * kNumCu) return kTileL;
+  return avg < 40 ? t : kTileM;
+}
+
+// Down projections of one or two experts of >= 32 MiB (an expert-parallel share): their column tiles
+// leave most CUs idle, so the K split fills the GPU (pick_down_split) and the tile holds a segment's rows
+// at least height.  One Mixtral-8x7B expert, bf16, down and plane sum, against 128x128 with K split 2
+// (cold, one box; us): 31 rows 90.8 -> 27.0 on 32x128 and 8 splits, 64 rows 96.2 -> 30.2 and 128 rows
+// 103.2 -> 39.3 on 64x128 (8, 4 splits), 256 / 512 / 1024 rows 100.5 / 105.5 / 140.3 -> 52.4 / 66.3 / 102.2
+// on 256x256 (8, 8, 4 splits); e4m3 weights 31 / 128 / 512 rows 60.4 / 85.9 / 89.5 -> 20.1 / 34.5 / 66.5.
+// Segments of a launch with several scatter, hence the lower bound of the 32-row tile there.
+// expert_bytes: at two bytes per weight, as the split is picked.
+bool few_large_down(int S, int N, double expert_bytes) {
+  return expert_bytes >= 32.0 * 1024 * 1024 && static_cast<long long>(S) * (N / 128) * 4 <= kNumCu;
+}
+int few_large_down_tile(int S, double avg) {
+  return avg < 0.7 ? kTileXS : avg <= (S == 1 ? 36 : 24) ? kTileS : avg <= 192 ? kTileMS : kTileL;
 }
 
 // Tile heuristic (the host knows only the row bound, or a caller's estimate, and the shapes).
@@ -2323,7 +2361,16 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
   const double expert_bytes = static_cast<double>(p.nb_rows) * p.K * p.k_split * (b_fp8 ? 1 : 2);
   const bool silu = epi_silu(epi);
   int t;
-  if (expert_bytes >= 32.0 * 1024 * 1024) {
+  bool idle_ok = false;   // a 256x256 choice that stands with fewer tiles than CUs
+  if (!b_fp8 && !silu && p.k_split > 1 && few_large_down(S, p.N, expert_bytes)) {
+    t = few_large_down_tile(S, avg);
+    idle_ok = true;   // the K split fills the CUs
+  } else if (!b_fp8 && silu && S == 1 && expert_bytes >= 32.0 * 1024 * 1024) {
+    // one expert: the rows are known, so the tile that holds them (Mixtral-8x7B, us, cold: 64 rows 62.3
+    // on 128x128, 51.5 on 64x128; 511 rows, four m-tiles of 128, 157 against 90 on 256x256)
+    t = avg < 0.7 ? kTileXS : avg <= 32 ? kTileS : avg <= 64 ? kTileMS : avg <= 128 ? kTileM : kTileL;
+    idle_ok = true;
+  } else if (expert_bytes >= 32.0 * 1024 * 1024) {
     // (W8A8 gate/up at 16 rows per expert on the routed, gathered rows of a Mixtral-8x7B
     // decode batch: 182 us on 32x128 tiles, 190 us streamed.  bf16 down projection on 128x128
     // with its K split 2, first from 4 expected rows: Mixtral-8x7B layers at 16 / 20 /
@@ -2346,6 +2393,11 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
     // then on 64x128 tiles (the ring) to 64 rows (104 / 128 / 160 / 192 / 224 / 240 tokens 470 / 480 /
     // 491 / 503 / 515 / 525 -> 438 / 449 / 457 / 469 / 480 / 517 us against 128x128)
     else if (silu) t = avg < 0.7 ? kTileXS : avg < 25 ? kTileS : avg < 64 ? kTileMS : kTileL;
+    // a launch as wide as a gate/up (four rounds of column tiles; no K split): the op point, 8 Mixtral-8x7B
+    // weights (28672 x 4096), one hot, cold, 8 / 31 / 64 / 128 / 256 / 512 rows 166 / 297 / 330 / 342 / 381 / 406 us
+    // on 128x128, 157 / 266 / 289 / 307 / 318 / 389 on 64x128, 171 / 308 / 324 / 329 / 308 / 333 on 256x256
+    else if (S >= 8 && p.k_split == 1 && static_cast<long long>(S) * (p.N / 128) >= 4 * kNumCu)
+      t = avg < 0.7 ? kTileXS : avg < 24 ? kTileMS : kTileL;
     else t = avg < 0.7 ? kTileXS : avg < 128 ? kTileM : kTileL;
   } else if (silu) {
     // From the row bound, not the expected rows: the Qwen3-30B-A3B 32-expert share at 2048
@@ -2359,9 +2411,14 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
   }
   if (t == kTileL) {
     // fewer 256x256 tiles than CUs (a dense shared-expert launch, say) leaves CUs idle: step down
-    const long long mt = static_cast<long long>(p.max_rows) / 256 + S;
+    // (one large expert, whose tiles are known: half as many; the Mixtral-8x7B down projection unsplit
+    // at 3000 rows, 192 tiles, 372 us on 128x128 and 258 on 256x256, at 2048 rows 238 and 236)
+    // Half as many also for the routed bf16 launches of small experts (figures at routed_small_gate_up_tile).
+    const bool one_large = S == 1 && expert_bytes >= 32.0 * 1024 * 1024;
+    const bool half = one_large || (!b_fp8 && S >= 8 && expert_bytes < 32.0 * 1024 * 1024);
+    const long long mt = (static_cast<long long>(p.max_rows) + (one_large ? 255 : 0)) / 256 + (one_large ? 0 : S);
     const int oc = gemm_out_cols_per_tile(kTileL, epi);
-    if (p.N % oc == 0 && mt * (p.N / oc) * p.k_split < kNumCu) t = kTileM;
+    if (!idle_ok && p.N % oc == 0 && mt * (p.N / oc) * p.k_split < (half ? kNumCu / 2 : kNumCu)) t = kTileM;
   }
   while (t != kTileXS && p.N % gemm_out_cols_per_tile(t, epi) != 0) t = tile_step_down(t);
   return t;
@@ -2392,15 +2449,23 @@ int gemm_choose_tile(const GemmArgs& p, int epi, bool b_fp8, bool a_fp8) {
     // 22.8 streamed, 768 tokens 29.7 / 27.3 on 64x128 against 39.8 / 36.2 on 128x128, 2048 tokens
     // 48.9 on 64x128 / 39.0 on 128x128 against 53.8 / 52.6 on 256x256; DeepSeek-V2-Lite 768 tokens
     // 108.8 / 66.9 on 64x128 against 125.9 / 78.9 on 128x128).
-    if (expert_bytes >= 32.0 * 1024 * 1024) {
+    // One large expert, whose rows are known: the gate/up on the tile that holds them (Mixtral-8x7B, cold,
+    // us: 31 rows 35.7 -> 29.8 on 32x128, 64 / 128 rows 44.2 / 53.7 -> 36.4 / 45.9 on 64x128).
+    const bool few_down = !epi_silu(epi) && p.k_split > 1 && few_large_down(p.S, p.N, 2.0 * expert_bytes);
+    if (few_down) {
+      tile = few_large_down_tile(p.S, avg);
+    } else if (expert_bytes >= 32.0 * 1024 * 1024 && epi_silu(epi) && p.S == 1) {
+      tile = avg < 1 ? kTileXS : avg <= 32 ? kTileS : avg <= 128 ? kTileMS : avg <= 256 ? kTileM : kTileL;
+    } else if (expert_bytes >= 32.0 * 1024 * 1024) {
       tile = avg < 1 ? kTileXS : avg < 24 ? kTileS : avg < 56 ? kTileMS : avg < 128 ? kTileM : kTileL;
     } else {
       tile = avg < 4 ? kTileXS : avg < 20 ? kTileS : avg < 100 ? kTileMS : avg < 256 ? (epi_silu(epi) ? kTileMS : kTileM)
                                                                                        : kTileL;
       keep_xs = avg >= 1;
     }
-    if (tile == kTileL && (static_cast<long long>(p.max_rows) / 256 + p.S) * (p.N / gemm_out_cols_per_tile(kTileL, epi)) *
-                                  p.k_split < kNumCu)
+    if (tile == kTileL && !few_down &&
+        (static_cast<long long>(p.max_rows) / 256 + p.S) * (p.N / gemm_out_cols_per_tile(kTileL, epi)) *
+                p.k_split < kNumCu)
       tile = kTileM;
     while (tile != kTileXS && p.N % gemm_out_cols_per_tile(tile, epi) != 0) tile = tile_step_down(tile);
   } else {

@@ -142,6 +142,9 @@ int stream_out_cols(int N, int epi, bool fp8);
 hipError_t launch_stream_gemm(const GemmArgs& p, int epi, int ops, int max_rows, int mblk, hipStream_t s);
 int gemm_out_cols_per_tile(int tile, int epi);
 double expected_m_tiles(double rows, int bm);
+// Down projections of one or two large experts, and the tile of their split launches.
+bool few_large_down(int S, int N, double expert_bytes);
+int few_large_down_tile(int S, double avg);
 // fp32 operands: A, B and the output in fp32 (epi kEpiSiluF32 or kEpiStoreF32); LDS-tiled kernels only
 // (tiles 128x128, 64x128 and 32x128 on the bf16 MFMA over three bf16 terms per operand, 16x64 on the
 // fp32 MFMA v_mfma_f32_16x16x4f32).

@@ -104,3 +104,35 @@ def test_op_point_merges_repeated_weights(dev, E, ep, K, N, pattern):
     ref = oracle.grouped_gemm(a, w * ep, blocks)
     # one bf16 rounding of the output, at most 2^-9 of each value; fp32 sums of up to 4096 terms
     assert oracle.rel_l2(out.cpu().float(), ref) <= 2.0 ** -8
+
+
+# One or two experts of 32 MiB and more, whose down projection splits K over the idle CUs: both sides of
+# each tile and split bound (32, 36, 64, 192 rows; 8, 4 and 2 splits), and routed small experts at the
+# bounds of the 64x128 and 256x256 tiles.
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,H,I,rows", [(1, 1024, 16384, r) for r in (1, 32, 33, 36, 37, 64, 65, 128, 192, 193, 257, 600)]
+                         + [(2, 1024, 16384, r) for r in (1, 49, 130, 400)]
+                         + [(16, 512, 1024, r) for r in (127, 128, 256, 639, 641, 3199, 3201)])
+@pytest.mark.parametrize("mode", ["bf16", "w8a16"])
+def test_experts_tile_bounds(dev, E, H, I, rows, mode):
+    g = torch.Generator().manual_seed(rows)
+    counts = torch.bincount(torch.randint(0, E, (rows,), generator=g), minlength=E)
+    x = torch.randn(rows, H, generator=g).to(torch.bfloat16)
+    wgu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(torch.bfloat16)
+    wd = (torch.randn(E, H, I, generator=g) * 0.05).to(torch.bfloat16)
+    ref_gu, ref_d, scales = wgu.float(), wd.float(), None
+    if mode == "w8a16":
+        (wgu, sgu), (wd, sd) = oracle.quantize_weights_fp8(wgu.float()), oracle.quantize_weights_fp8(wd.float())
+        ref_gu, ref_d = wgu.float() * sgu[..., None], wd.float() * sd[..., None]
+        scales = (sgu.to(dev), sd.to(dev))
+    print("CASE", dict(E=E, H=H, I=I, rows=rows, mode=mode), flush=True)
+    y = ops.experts(x.to(dev), wgu.to(dev), wd.to(dev), counts.to(torch.int32).to(dev), E, scales)
+    xd, rgu, rd = x.to(dev).float(), ref_gu.to(dev), ref_d.to(dev)
+    ref, r = torch.empty(rows, H, device=dev), 0
+    for e, c in enumerate(counts.tolist()):
+        gu = xd[r:r + c] @ rgu[e].T
+        h = (torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]).to(torch.bfloat16).float()
+        ref[r:r + c] = h @ rd[e].T
+        r += c
+    # one bf16 rounding of the output and of h, each at most 2^-9 of a value
+    assert oracle.rel_l2(y.cpu().float(), ref.cpu()) <= 2.0 ** -8
