@@ -84,34 +84,48 @@ __global__ __launch_bounds__(kAlignMbThreads) void align_place_kernel(
   for (int i = tid; i < kAlignMbWaves * n_loc; i += kAlignMbThreads) hist[i] = 0;
   for (int e = tid; e < n_loc; e += kAlignMbThreads) tot[e] = base[e] = 0;
   __syncthreads();
-  // Column sums of the chunk-count matrix (at most kAlignMbMaxCells cells, coalesced;
-  // integer LDS atomics, so the order does not matter): totals, and the chunks before this
-  // one.  The first few cells per thread are loaded before the recount below, so their
-  // latency overlaps it.
-  const int cells = static_cast<int>(gridDim.x) * n_loc;
-  const int own = static_cast<int>(blockIdx.x) * n_loc;
-  constexpr int kEarly = 4;
+  // Column sums of the chunk-count matrix (at most kAlignMbMaxCells cells, coalesced): totals, and the
+  // chunks before this one.  A thread sums one expert's cells of every groups-th chunk in registers and
+  // adds them to LDS once (integers, so the order does not matter).  The first few cells per thread are
+  // loaded before the recount below, so their latency overlaps it.
+  const int rows = static_cast<int>(gridDim.x);
+  const int own = static_cast<int>(blockIdx.x);
+  const int cols = min(n_loc, kAlignMbThreads);
+  const int groups = kAlignMbThreads / cols;
+  const int col = tid % cols;
+  const int r0 = tid / cols < groups ? tid / cols : rows;
+  constexpr int kEarly = 8;
   int early[kEarly];
 #pragma unroll
   for (int j = 0; j < kEarly; ++j) {
-    const int i = tid + j * kAlignMbThreads;
-    early[j] = i < cells ? hist_g[i] : 0;
+    const int r = r0 + j * groups;
+    early[j] = r < rows ? hist_g[r * n_loc + col] : 0;
   }
   const int sub = chunk / kAlignMbWaves;
   const long long beg = static_cast<long long>(blockIdx.x) * chunk + static_cast<long long>(w) * sub;
   const int b0 = static_cast<int>(min<long long>(beg, N));
   const int b1 = static_cast<int>(min<long long>(beg + sub, N));
   count_slice<false>(ids, b0, b1, e_lo, n_loc, nbits, hist + w * n_loc);
-  auto add_cell = [&](int i, int c) {
-    if (c != 0) {
-      atomicAdd(&tot[i % n_loc], c);
-      if (i < own) atomicAdd(&base[i % n_loc], c);
-    }
-  };
+  for (int e = col; e < n_loc; e += cols) {
+    int t = 0, before = 0;
+    int r = r0;
+    if (e == col) {
 #pragma unroll
-  for (int j = 0; j < kEarly; ++j) add_cell(tid + j * kAlignMbThreads, early[j]);
-#pragma unroll 4
-  for (int i = tid + kEarly * kAlignMbThreads; i < cells; i += kAlignMbThreads) add_cell(i, hist_g[i]);
+      for (int j = 0; j < kEarly; ++j) {
+        t += early[j];
+        before += r0 + j * groups < own ? early[j] : 0;
+      }
+      r += kEarly * groups;
+    }
+#pragma unroll 8
+    for (; r < rows; r += groups) {
+      const int c = hist_g[r * n_loc + e];
+      t += c;
+      before += r < own ? c : 0;
+    }
+    if (t != 0) atomicAdd(&tot[e], t);
+    if (before != 0) atomicAdd(&base[e], before);
+  }
   __syncthreads();
   scan_experts(tot, n_loc, offs);
   __syncthreads();

@@ -19,21 +19,37 @@ __device__ __forceinline__ float dpp_f(float v) {
   return __int_as_float(dpp_i<CTRL>(__float_as_int(v)));
 }
 
-__device__ __forceinline__ void take_better(float& bv, int& bi, float ov, int oi) {
-  if (ov > bv || (ov == bv && oi < bi)) {
-    bv = ov;
-    bi = oi;
-  }
+template <int LPT>
+__device__ __forceinline__ uint32_t group_max_u32(uint32_t v) {
+  if constexpr (LPT >= 2) v = max(v, static_cast<uint32_t>(dpp_i<0xB1>(static_cast<int>(v))));     // quad_perm [1,0,3,2]
+  if constexpr (LPT >= 4) v = max(v, static_cast<uint32_t>(dpp_i<0x4E>(static_cast<int>(v))));     // quad_perm [2,3,0,1]
+  if constexpr (LPT >= 8) v = max(v, static_cast<uint32_t>(dpp_i<0x141>(static_cast<int>(v))));    // row_half_mirror
+  if constexpr (LPT >= 16) v = max(v, static_cast<uint32_t>(dpp_i<0x140>(static_cast<int>(v))));   // row_mirror
+#pragma unroll
+  for (int m = 16; m < LPT; m <<= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), m, LPT)));
+  return v;
 }
 
 template <int LPT>
-__device__ __forceinline__ void group_argmax(float& bv, int& bi) {
-  if constexpr (LPT >= 2) take_better(bv, bi, dpp_f<0xB1>(bv), dpp_i<0xB1>(bi));     // quad_perm [1,0,3,2]
-  if constexpr (LPT >= 4) take_better(bv, bi, dpp_f<0x4E>(bv), dpp_i<0x4E>(bi));     // quad_perm [2,3,0,1]
-  if constexpr (LPT >= 8) take_better(bv, bi, dpp_f<0x141>(bv), dpp_i<0x141>(bi));   // row_half_mirror
-  if constexpr (LPT >= 16) take_better(bv, bi, dpp_f<0x140>(bv), dpp_i<0x140>(bi));  // row_mirror
+__device__ __forceinline__ int group_min_i32(int v) {
+  if constexpr (LPT >= 2) v = min(v, dpp_i<0xB1>(v));
+  if constexpr (LPT >= 4) v = min(v, dpp_i<0x4E>(v));
+  if constexpr (LPT >= 8) v = min(v, dpp_i<0x141>(v));
+  if constexpr (LPT >= 16) v = min(v, dpp_i<0x140>(v));
 #pragma unroll
-  for (int m = 16; m < LPT; m <<= 1) take_better(bv, bi, __shfl_xor(bv, m, LPT), __shfl_xor(bi, m, LPT));
+  for (int m = 16; m < LPT; m <<= 1) v = min(v, __shfl_xor(v, m, LPT));
+  return v;
+}
+
+// Keys that order as the logits do (the two zeros equal), above 0 for every value that can be picked;
+// NaN gets 0.
+__device__ __forceinline__ uint32_t pick_key(float x) {
+  const uint32_t u = __float_as_uint(x + 0.f);
+  const uint32_t key = u ^ (static_cast<uint32_t>(static_cast<int>(u) >> 31) | 0x80000000u);
+  return x == x ? key : 0u;
+}
+__device__ __forceinline__ float pick_value(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
 }
 
 template <int LPT>
@@ -67,13 +83,13 @@ __device__ __forceinline__ void route_rows(const float* __restrict__ logits, int
     const int t = t0 + sub;
     const bool tv = t < T;
     float v[VPL];
-    uint32_t avail = 0;
+    uint32_t key[VPL];   // 0: no value, or picked
 #pragma unroll
     for (int j = 0; j < VPL; ++j) {
       const int e = li + j * LPT;
       const bool ok = tv && e < E;
       v[j] = ok ? logits[static_cast<long long>(t) * E + e] : NEG_INF;
-      if (ok) avail |= 1u << j;
+      key[j] = ok ? pick_key(v[j]) : 0u;
     }
     // Pick r lives in lane r % LPT of the group (slot r / LPT), so the rounds form a rolled
     // loop: the kernel stays a few hundred instructions, which matters when it runs from a
@@ -88,19 +104,18 @@ __device__ __forceinline__ void route_rows(const float* __restrict__ logits, int
     float mx = NEG_INF;
 #pragma unroll 1
     for (int r = 0; r < k; ++r) {
-      float bv = NEG_INF;
-      int bi = 0x7fffffff;
-      // Selects, no branches: written with && / || the compiler made each value a divergent
-      // branch block (eight per round at 128 experts), ~0.65 us per pick (timestamped: top-8 of
-      // 128 took 5.3 us of the Qwen3-shape route+align kernel).
+      // The largest key, then the lowest id that holds it: integer maxima and minima, where comparing
+      // (value, id) pairs was a chain of ~8 dependent selects per value (0.44 us a pick at 128 experts).
+      uint32_t m = 0;
 #pragma unroll
-      for (int j = 0; j < VPL; ++j) {
-        const int e = li + j * LPT;
-        const bool better = (((avail >> j) & 1u) != 0) & ((v[j] > bv) | ((v[j] == bv) & (e < bi)));
-        bv = better ? v[j] : bv;
-        bi = better ? e : bi;
-      }
-      group_argmax<LPT>(bv, bi);
+      for (int j = 0; j < VPL; ++j) m = max(m, key[j]);
+      m = group_max_u32<LPT>(m);
+      int bi = 0x7fffffff;
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) bi = min(bi, key[j] == m ? li + j * LPT : 0x7fffffff);
+      bi = group_min_i32<LPT>(bi);
+      bi = m != 0 ? bi : 0x7fffffff;
+      const float bv = m != 0 ? pick_value(m) : NEG_INF;
       if (r == 0) mx = bv;
       if (r % LPT == li) {
 #pragma unroll
@@ -110,7 +125,8 @@ __device__ __forceinline__ void route_rows(const float* __restrict__ logits, int
             myi[j] = bi;
           }
       }
-      if (bi != 0x7fffffff && (bi % LPT) == li) avail &= ~(1u << (bi / LPT));
+#pragma unroll
+      for (int j = 0; j < VPL; ++j) key[j] = li + j * LPT == bi ? 0u : key[j];
     }
     float ex[KPL];
     float part = 0.f;
@@ -382,6 +398,60 @@ __device__ __forceinline__ void align_tiny(const int32_t* __restrict__ ids, int 
     if (p >= 0) {
       sorted_flat[p] = lane;
       sorted_tok[p] = lane / k;
+    }
+  }
+}
+
+// The same sort where each of the workgroup's waves has at most one row of 64 ids and a lane can hold an
+// expert (N <= kAlignThreads, n_loc <= 64): one match mask per id, one barrier (each wave sums the other
+// waves' counts for itself and scans the experts in registers).  lds: kAlignWaves * n_loc ints, zeroed
+// before a barrier by the caller.  Same outputs as align_rows.
+__device__ __forceinline__ void align_row_per_wave(const int32_t* __restrict__ ids, int N, int k, int e_lo, int n_loc,
+                                                   int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+                                                   int32_t* __restrict__ sorted_flat, int32_t* __restrict__ sorted_tok,
+                                                   int32_t* __restrict__ pos, int* lds) {
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+  const int nw = (N + 63) / 64;
+  const int i = w * 64 + lane;
+  const int nbits = n_loc > 1 ? 32 - __clz(n_loc - 1) : 0;
+  int e = -1;
+  uint64_t m = 0;
+  if (w < nw) {
+    if (i < N) {
+      const int g = ids[i] - e_lo;
+      e = (g >= 0 && g < n_loc) ? g : -1;
+    }
+    m = match_mask(e < 0 ? 0 : e, nbits, __ballot(e >= 0));
+    if (e >= 0 && lane == __ffsll(static_cast<unsigned long long>(m)) - 1) lds[w * n_loc + e] = __popcll(m);
+  }
+  __syncthreads();
+  if (w >= nw) return;
+  int tot = 0, before = 0;
+  if (lane < n_loc) {
+#pragma unroll 4
+    for (int ww = 0; ww < nw; ++ww) {
+      const int c = lds[ww * n_loc + lane];
+      tot += c;
+      before += ww < w ? c : 0;
+    }
+  }
+  const int incl = wave_incl_scan(tot);
+  const int first = __shfl(incl - tot + before, e < 0 ? 0 : e, 64);
+  if (w == 0) {
+    if (lane < n_loc) {
+      counts[lane] = tot;
+      offsets[lane] = incl - tot;
+    }
+    if (lane == 63) offsets[n_loc] = incl;
+  }
+  if (i < N) {
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int p = e >= 0 ? first + __popcll(m & lt_mask) : -1;
+    pos[i] = p;
+    if (p >= 0) {
+      sorted_flat[p] = i;
+      sorted_tok[p] = i / k;
     }
   }
 }
