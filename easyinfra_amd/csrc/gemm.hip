@@ -2459,8 +2459,19 @@ int gemm_choose_tile(const GemmArgs& p, int epi, bool b_fp8, bool a_fp8) {
     } else if (expert_bytes >= 32.0 * 1024 * 1024) {
       tile = avg < 1 ? kTileXS : avg < 24 ? kTileS : avg < 56 ? kTileMS : avg < 128 ? kTileM : kTileL;
     } else {
-      tile = avg < 4 ? kTileXS : avg < 20 ? kTileS : avg < 100 ? kTileMS : avg < 256 ? (epi_silu(epi) ? kTileMS : kTileM)
-                                                                                       : kTileL;
+      // (segments an eighth of which hold 8 times the rows of the others, rows per segment in brackets: gate/up,
+      // Qwen3 share 4100 / 8192 rows [128 / 256] 60.5 / 103.3 on 64x128, 60.2 / 79.8 on 128x128, 49.1 / 91.1 on
+      // 256x256, 16 DeepSeek-V2-Lite experts 2048 / 4100 rows 60.5 / 101.9, 60.0 / 66.8 and 49.6 / 90.8, 32 of them
+      // 4100 / 8192 rows 104.9 / 188.5, 87.9 / 129.1 and 89.4 / 138.0; down, 1024 rows [32] 21.6 -> 16.9 and 29.7 -> 23.8
+      // on 32x128 against 64x128)
+      const bool one_round = static_cast<long long>(p.S) * (p.N / 128) * 5 <= 4 * kNumCu;   // of 256x256 gate/up tiles
+      // (64 DeepSeek-V2-Lite experts, layers: 2400 tokens [225] 593 -> 476 us on 128x128, 3300 [309] 550 -> 568)
+      const bool two_rounds = static_cast<long long>(p.S) * (p.N / 128) >= 2 * kNumCu;
+      if (epi_silu(epi))
+        tile = avg < 4 ? kTileXS : avg < 20 ? kTileS : avg < 100 ? kTileMS : avg < 200 && one_round ? kTileL
+               : avg < (two_rounds ? 256 : 384) ? kTileM : kTileL;
+      else
+        tile = avg < 4 ? kTileXS : avg < 40 ? kTileS : avg < 100 ? kTileMS : avg < 256 ? kTileM : kTileL;
       keep_xs = avg >= 1;
     }
     if (tile == kTileL && !few_down &&
