@@ -2289,18 +2289,11 @@ int gemm_out_cols_per_tile(int tile, int epi) {
 // 54.9 / 70.5, 45.9 / 50.2 / 73.0 and 43.9 / 41.7 / 44.1.  A 256x256 tile takes about the same time whatever
 // its height, so it wins once the rows would need a second round of the small tiles, down to half a
 // round of tiles.
-static int routed_small_gate_up_tile(const GemmArgs& p, int S, double avg, int t, bool fp8) {
+static int routed_small_gate_up_tile(const GemmArgs& p, int S, double avg, int t) {
   const long long tiles_l = static_cast<long long>(S) * static_cast<long long>((avg + 255) / 256) * (p.N / 128);
-  const long long tiles_ms = static_cast<long long>(S) * static_cast<long long>((avg + 63) / 64) * (p.N / 64);
   const long long tiles_m = static_cast<long long>(S) * static_cast<long long>((avg + 127) / 128) * (p.N / 64);
-  if (!fp8) {
-    if (avg >= 40 && tiles_l >= kNumCu / 2) return kTileL;
-    return avg >= (tiles_m >= 2 * kNumCu ? 8 : 16) && avg < 64 ? kTileMS : t;
-  }
-  if (avg >= 40 && tiles_l >= kNumCu) return kTileL;
-  if (avg >= 20 && avg < 64 && tiles_ms <= 3 * kNumCu) return kTileMS;
-  if (avg >= 8 && avg < 20 && tiles_m >= 2 * kNumCu) return kTileM;
-  return t;
+  if (avg >= 40 && tiles_l >= kNumCu / 2) return kTileL;
+  return avg >= (tiles_m >= 2 * kNumCu ? 8 : 16) && avg < 64 ? kTileMS : t;
 }
 
 // e4m3 (W8A8) tiles do half the MFMA work per weight byte: the 64x128 band reaches to 80 rows, the
@@ -2321,9 +2314,11 @@ static int routed_small_down_tile(const GemmArgs& p, int S, double avg, int t, b
     if ((tiles_l >= kNumCu / 2 && tiles_l * 5 <= kNumCu * 4) || tiles_l >= 2 * kNumCu || avg >= 200) return kTileL;
     return avg < 72 ? kTileMS : kTileM;
   }
-  if (avg >= 20 && avg < 80 && tiles_ms <= 3 * kNumCu) return kTileMS;   // one round of 64x128 workgroups
-  if (avg >= 64 && tiles_l >= 2 * kNumCu) return kTileL;
-  return avg < 40 ? t : kTileM;
+  // W8A8: 64 DeepSeek-V2-Lite experts 1500 / 3000 / 6000 / 9000 rows [23 / 47 / 94 / 141] 45.2 / 51.9 / 67.1 / 82.4, 46.0 /
+  // 55.4 / 55.3 / 63.7 and 46.1 / 49.4 / 65.2 / 64.5, Qwen3 share 8192 rows [256] 38.5, 40.7 and 32.2
+  if (avg >= 200 || (avg >= 130 && tiles_l >= 2 * kNumCu)) return kTileL;
+  if (avg >= 20 && avg < (tiles_ms <= 3 * kNumCu ? 80 : 60)) return kTileMS;   // 80: one round of 64x128 workgroups
+  return avg < 20 ? t : kTileM;
 }
 
 // Down projections of one or two experts of >= 32 MiB (an expert-parallel share): their column tiles
@@ -2404,7 +2399,7 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
     // tokens (~3900 local rows, 56-551 per expert) measured 72 us on 256x256 tiles and 89 us on
     // 128x128 (the expected 125 rows per expert would pick the latter).
     t = avg_bound >= 256 ? kTileL : avg_bound >= 96 ? kTileM : avg_bound >= 24 ? kTileS : kTileXS;
-    if (S >= 8 && avg_bound < 256) t = routed_small_gate_up_tile(p, S, avg, t, b_fp8);
+    if (S >= 8 && avg_bound < 256) t = routed_small_gate_up_tile(p, S, avg, t);
   } else {
     t = avg < 6 ? kTileXS : avg < 96 ? kTileS : avg < 384 ? kTileM : kTileL;
     if (S >= 8 && avg >= (b_fp8 ? 20 : 8) && avg < 384) t = routed_small_down_tile(p, S, avg, t, b_fp8);
@@ -2413,9 +2408,9 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
     // fewer 256x256 tiles than CUs (a dense shared-expert launch, say) leaves CUs idle: step down
     // (one large expert, whose tiles are known: half as many; the Mixtral-8x7B down projection unsplit
     // at 3000 rows, 192 tiles, 372 us on 128x128 and 258 on 256x256, at 2048 rows 238 and 236)
-    // Half as many also for the routed bf16 launches of small experts (figures at routed_small_gate_up_tile).
+    // Half as many also for the routed launches of small experts (figures at routed_small_gate_up_tile).
     const bool one_large = S == 1 && expert_bytes >= 32.0 * 1024 * 1024;
-    const bool half = one_large || (!b_fp8 && S >= 8 && expert_bytes < 32.0 * 1024 * 1024);
+    const bool half = one_large || ((silu || !b_fp8) && S >= 8 && expert_bytes < 32.0 * 1024 * 1024);
     const long long mt = (static_cast<long long>(p.max_rows) + (one_large ? 255 : 0)) / 256 + (one_large ? 0 : S);
     const int oc = gemm_out_cols_per_tile(kTileL, epi);
     if (!idle_ok && p.N % oc == 0 && mt * (p.N / oc) * p.k_split < (half ? kNumCu / 2 : kNumCu)) t = kTileM;
@@ -2465,13 +2460,16 @@ int gemm_choose_tile(const GemmArgs& p, int epi, bool b_fp8, bool a_fp8) {
       // 4100 / 8192 rows 104.9 / 188.5, 87.9 / 129.1 and 89.4 / 138.0; down, 1024 rows [32] 21.6 -> 16.9 and 29.7 -> 23.8
       // on 32x128 against 64x128)
       const bool one_round = static_cast<long long>(p.S) * (p.N / 128) * 5 <= 4 * kNumCu;   // of 256x256 gate/up tiles
-      // (64 DeepSeek-V2-Lite experts, layers: 2400 tokens [225] 593 -> 476 us on 128x128, 3300 [309] 550 -> 568)
+      // (64 DeepSeek-V2-Lite experts, layers: 2400 tokens [225] 593 -> 476 us on 128x128, 3300 [309] 550 -> 568;
+      // gate/up 1500 / 3000 / 6000 rows [23 / 47 / 94] 83.2 / 105.7 / 169.5 on 32x128, 103.9 / 115.9 / 148.6 on 64x128, 103.0 /
+      // 123.9 / 126.5 on 128x128; down 4600 / 6000 rows [72 / 94] 81.1 / 93.3 on 64x128, 73.6 / 73.5 on 128x128)
       const bool two_rounds = static_cast<long long>(p.S) * (p.N / 128) >= 2 * kNumCu;
+      const bool wide = static_cast<long long>(p.S) * (p.N / 128) >= 4 * kNumCu;
       if (epi_silu(epi))
-        tile = avg < 4 ? kTileXS : avg < 20 ? kTileS : avg < 100 ? kTileMS : avg < 200 && one_round ? kTileL
-               : avg < (two_rounds ? 256 : 384) ? kTileM : kTileL;
+        tile = avg < 4 ? kTileXS : avg < (two_rounds ? 56 : 20) ? kTileS : avg < (two_rounds ? 56 : 100) ? kTileMS
+               : avg < 200 && one_round ? kTileL : avg < (two_rounds ? 256 : 384) ? kTileM : kTileL;
       else
-        tile = avg < 4 ? kTileXS : avg < 40 ? kTileS : avg < 100 ? kTileMS : avg < 256 ? kTileM : kTileL;
+        tile = avg < 4 ? kTileXS : avg < 40 ? kTileS : avg < (wide ? 60 : 100) ? kTileMS : avg < 256 ? kTileM : kTileL;
       keep_xs = avg >= 1;
     }
     if (tile == kTileL && !few_down &&
