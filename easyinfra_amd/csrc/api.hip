@@ -112,9 +112,8 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
   // the tile the launch will take (the W8A16 layer is costed as bf16: its workspace query does not
   // see the weight type; any split chosen here is valid for it, at worst on its LDS tiles)
   int tile = gemm_choose_tile(q, kEpiStoreF32, w8a8, w8a8);
-  if (!w8a8 && tile != kTileStream && few_large_down(n_local, H, static_cast<double>(H) * I * 2))
-    tile = few_large_down_tile(n_local, static_cast<double>(rows_hint > 0 ? std::min(rows_hint, max_rows) : max_rows) /
-                                            n_local);
+  const bool few_large = rows_hint <= 0 && !w8a8 && few_large_down(n_local, H, static_cast<double>(H) * I * 2);
+  if (few_large && tile != kTileStream) tile = few_large_down_tile(n_local, static_cast<double>(max_rows) / n_local);
   if (tile == kTileStream) {
     // Few rows per segment: the weight-streaming kernel runs one workgroup per (segment,
     // column group, 32-row chunk, split).  Split until there are about 6 workgroups per CU
@@ -144,7 +143,7 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
     // one or two experts: split until there is a workgroup per CU (figures at few_large_down)
     const long long wgs = static_cast<long long>(segs * std::ceil(per / bm)) * (H / bn);
     int split = 2;
-    while (split < 8 && wgs * split * 2 <= kNumCu && steps % (split * 2) == 0) split *= 2;
+    while (few_large && split < 8 && wgs * split * 2 <= kNumCu && steps % (split * 2) == 0) split *= 2;
     return split;
   }
   if (w8a8) I /= 2;   // e4m3 tiles run at twice the bf16 rate: cost them as half the K
@@ -188,8 +187,10 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
     double cost = rounds / split * t_tile + (split - 1) * t_plane;
     // too few workgroups to fill the GPU: twice over for the one-tile-per-workgroup kernels, once
     // for the persistent 256x256 one (whose workgroups walk their tiles)
-    // (one expert: three quarters, 1500 Mixtral-8x7B rows 177 us with 4 splits, 148 with 2)
-    const bool few = tile == kTileL ? work * split < (one_seg ? 0.75 : 1.0) * kNumCu : items < 2 * kNumCu;
+    // (one expert: three quarters, 1500 Mixtral-8x7B rows 177 us with 4 splits, 148 with 2; routed small
+    // experts: under half, the least for which gemm_pick_tile takes 256x256)
+    const double fill = one_seg ? 0.75 : n_local >= 8 && expert_bytes < 32.0 * 1024 * 1024 ? 0.4 : 1.0;
+    const bool few = tile == kTileL ? work * split < fill * kNumCu : items < 2 * kNumCu;
     if (few && split < 8 && I % (128 * split) == 0) cost = 1e300;
     if (cost < best_cost * 0.98) {
       best_cost = cost;

@@ -2311,12 +2311,12 @@ static int routed_small_down_tile(const GemmArgs& p, int S, double avg, int t, b
     // (below 12 rows the two are level, 18.4 each at 4 rows and 21.2 at 8, unless 128x128 makes no more tiles than
     // CUs: 16 experts, 128 rows 23.9 -> 17.9 us; the Qwen3 share's layer at 128 tokens is 2 us slower on 64x128)
     if (avg < 40) return avg >= 12 || static_cast<long long>(S) * (p.N / 128) <= kNumCu ? kTileMS : kTileM;
-    if ((tiles_l >= kNumCu / 2 && tiles_l * 5 <= kNumCu * 4) || tiles_l >= 2 * kNumCu || avg >= 200) return kTileL;
+    if (tiles_l >= kNumCu / 2 && (tiles_l * 5 <= kNumCu * 4 || tiles_l >= 2 * kNumCu || avg >= 200)) return kTileL;
     return avg < 72 ? kTileMS : kTileM;
   }
   // W8A8: 64 DeepSeek-V2-Lite experts 1500 / 3000 / 6000 / 9000 rows [23 / 47 / 94 / 141] 45.2 / 51.9 / 67.1 / 82.4, 46.0 /
   // 55.4 / 55.3 / 63.7 and 46.1 / 49.4 / 65.2 / 64.5, Qwen3 share 8192 rows [256] 38.5, 40.7 and 32.2
-  if (avg >= 200 || (avg >= 130 && tiles_l >= 2 * kNumCu)) return kTileL;
+  if (tiles_l >= kNumCu / 2 && (avg >= 200 || (avg >= 130 && tiles_l >= 2 * kNumCu))) return kTileL;
   if (avg >= 20 && avg < (tiles_ms <= 3 * kNumCu ? 80 : 60)) return kTileMS;   // 80: one round of 64x128 workgroups
   return avg < 20 ? t : kTileM;
 }
@@ -2327,7 +2327,8 @@ static int routed_small_down_tile(const GemmArgs& p, int S, double avg, int t, b
 // (cold, one box; us): 31 rows 90.8 -> 27.0 on 32x128 and 8 splits, 64 rows 96.2 -> 30.2 and 128 rows
 // 103.2 -> 39.3 on 64x128 (8, 4 splits), 256 / 512 / 1024 rows 100.5 / 105.5 / 140.3 -> 52.4 / 66.3 / 102.2
 // on 256x256 (8, 8, 4 splits); e4m3 weights 31 / 128 / 512 rows 60.4 / 85.9 / 89.5 -> 20.1 / 34.5 / 66.5.
-// Segments of a launch with several scatter, hence the lower bound of the 32-row tile there.
+// Segments of a launch with several scatter, hence the lower bound of the 32-row tile there.  Not in the
+// fused layer, whose workspace keeps its two planes.
 // expert_bytes: at two bytes per weight, as the split is picked.
 bool few_large_down(int S, int N, double expert_bytes) {
   return expert_bytes >= 32.0 * 1024 * 1024 && static_cast<long long>(S) * (N / 128) * 4 <= kNumCu;
@@ -2357,10 +2358,11 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
   const bool silu = epi_silu(epi);
   int t;
   bool idle_ok = false;   // a 256x256 choice that stands with fewer tiles than CUs
-  if (!b_fp8 && !silu && p.k_split > 1 && few_large_down(S, p.N, expert_bytes)) {
+  const bool known = p.rows_hint <= 0;   // the row bound is the rows, not a layer's expectation
+  if (!b_fp8 && !silu && known && p.k_split > 1 && few_large_down(S, p.N, expert_bytes)) {
     t = few_large_down_tile(S, avg);
     idle_ok = true;   // the K split fills the CUs
-  } else if (!b_fp8 && silu && S == 1 && expert_bytes >= 32.0 * 1024 * 1024) {
+  } else if (!b_fp8 && silu && known && S == 1 && expert_bytes >= 32.0 * 1024 * 1024) {
     // one expert: the rows are known, so the tile that holds them (Mixtral-8x7B, us, cold: 64 rows 62.3
     // on 128x128, 51.5 on 64x128; 511 rows, four m-tiles of 128, 157 against 90 on 256x256)
     t = avg < 0.7 ? kTileXS : avg <= 32 ? kTileS : avg <= 64 ? kTileMS : avg <= 128 ? kTileM : kTileL;
@@ -2409,8 +2411,8 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
     // (one large expert, whose tiles are known: half as many; the Mixtral-8x7B down projection unsplit
     // at 3000 rows, 192 tiles, 372 us on 128x128 and 258 on 256x256, at 2048 rows 238 and 236)
     // Half as many also for the routed launches of small experts (figures at routed_small_gate_up_tile).
-    const bool one_large = S == 1 && expert_bytes >= 32.0 * 1024 * 1024;
-    const bool half = one_large || ((silu || !b_fp8) && S >= 8 && expert_bytes < 32.0 * 1024 * 1024);
+    const bool one_large = known && S == 1 && expert_bytes >= 32.0 * 1024 * 1024;
+    const bool half = one_large || ((silu || !b_fp8) && S >= 8 && avg < 384 && expert_bytes < 32.0 * 1024 * 1024);
     const long long mt = (static_cast<long long>(p.max_rows) + (one_large ? 255 : 0)) / 256 + (one_large ? 0 : S);
     const int oc = gemm_out_cols_per_tile(kTileL, epi);
     if (!idle_ok && p.N % oc == 0 && mt * (p.N / oc) * p.k_split < (half ? kNumCu / 2 : kNumCu)) t = kTileM;
@@ -2446,10 +2448,11 @@ int gemm_choose_tile(const GemmArgs& p, int epi, bool b_fp8, bool a_fp8) {
     // 108.8 / 66.9 on 64x128 against 125.9 / 78.9 on 128x128).
     // One large expert, whose rows are known: the gate/up on the tile that holds them (Mixtral-8x7B, cold,
     // us: 31 rows 35.7 -> 29.8 on 32x128, 64 / 128 rows 44.2 / 53.7 -> 36.4 / 45.9 on 64x128).
-    const bool few_down = !epi_silu(epi) && p.k_split > 1 && few_large_down(p.S, p.N, 2.0 * expert_bytes);
+    const bool known = p.rows_hint <= 0;
+    const bool few_down = !epi_silu(epi) && known && p.k_split > 1 && few_large_down(p.S, p.N, 2.0 * expert_bytes);
     if (few_down) {
       tile = few_large_down_tile(p.S, avg);
-    } else if (expert_bytes >= 32.0 * 1024 * 1024 && epi_silu(epi) && p.S == 1) {
+    } else if (expert_bytes >= 32.0 * 1024 * 1024 && epi_silu(epi) && known && p.S == 1) {
       tile = avg < 1 ? kTileXS : avg <= 32 ? kTileS : avg <= 128 ? kTileMS : avg <= 256 ? kTileM : kTileL;
     } else if (expert_bytes >= 32.0 * 1024 * 1024) {
       tile = avg < 1 ? kTileXS : avg < 24 ? kTileS : avg < 56 ? kTileMS : avg < 128 ? kTileM : kTileL;

@@ -97,6 +97,8 @@ struct RouteHistPlan {
 // measured against the router + two-pass align (one box, cache-cold layers): Qwen3-30B-A3B
 // 32-expert share at 256 and 600 tokens (512 and 1216 cells) 89.0 -> 86.7 and 105.9 -> 101.7
 // us, at 2048 tokens (4096 cells) equal, DeepSeek-V2-Lite 4096 tokens (16384 cells) 611 -> 620 us.
+// Twice as many with workgroups of 16 waves, in place of the separate histogram launch: DeepSeek-V2-Lite
+// 1200 / 4096 tokens 346 / 641 -> 340 / 637 us (with the other changes to the routing kernels).
 constexpr long long kRouteHistMaxCells = 2048;
 
 // Workgroups of 4 waves, or of 8 where that keeps the matrix within bounds (the Qwen3-30B-A3B
