@@ -307,15 +307,22 @@ __device__ __forceinline__ void mma_f32(f32x4_t (&acc)[MBE][G::NB], const bf16x8
   }
 }
 
+// a |= b | c, in one instruction and where it stands: the compiler would gather a slab's into one tree and
+// keep all their operands (up to 64 registers a lane) until then.
+__device__ __forceinline__ void or3(uint32_t& a, uint32_t b, uint32_t c) {
+  asm("v_or3_b32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+}
+
 // fp32 operands as three bf16 terms on the bf16 MFMA: x = hi + mid + lo, each the upper half of what
 // the terms before it leave.  A fp32 mantissa has 24 bits and each term takes 8, so the three hold x
-// exactly (down to terms below 2^-133).  Lane group q's eight values of a 32-wide k slab are the
-// 16-byte chunks q and q + 4 of the row, for A and B alike.
+// exactly while lo stays above the smallest bf16 (2^-133: operands down to 2^-109, and smaller ones whose
+// bits end in time).  `lost` collects what does not fit, in its lower half.  Lane group q's eight values of
+// a 32-wide k slab are the 16-byte chunks q and q + 4 of the row, for A and B alike.
 struct Split3 {
   bf16x8_t t[3];   // hi, mid, lo
 };
 
-__device__ __forceinline__ Split3 split3(const f32x4_t& c0, const f32x4_t& c1) {
+__device__ __forceinline__ Split3 split3(const f32x4_t& c0, const f32x4_t& c1, uint32_t& lost) {
   u32x4_t w[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -325,6 +332,10 @@ __device__ __forceinline__ Split3 split3(const f32x4_t& c0, const f32x4_t& c1) {
     for (int k = 0; k < 3; ++k) {
       const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
       w[k][i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);   // the upper halves
+      if (k == 2) {
+        or3(lost, u0, u1);
+        break;
+      }
       x0 -= __uint_as_float(u0 & 0xffff0000u);
       x1 -= __uint_as_float(u1 & 0xffff0000u);
     }
@@ -333,9 +344,9 @@ __device__ __forceinline__ Split3 split3(const f32x4_t& c0, const f32x4_t& c1) {
                  __builtin_bit_cast(bf16x8_t, w[2])}};
 }
 
-__device__ __forceinline__ Split3 split3_lds(const uint16_t* s, int R, int q) {
+__device__ __forceinline__ Split3 split3_lds(const uint16_t* s, int R, int q, uint32_t& lost) {
   return split3(*reinterpret_cast<const f32x4_t*>(&s[R * 64 + ((q ^ swz(R)) << 3)]),
-                *reinterpret_cast<const f32x4_t*>(&s[R * 64 + (((q + 4) ^ swz(R)) << 3)]));
+                *reinterpret_cast<const f32x4_t*>(&s[R * 64 + (((q + 4) ^ swz(R)) << 3)]), lost);
 }
 
 // One row of fragments times all columns: the six products above 2^-22 of x*y, smallest first.
@@ -353,31 +364,27 @@ __device__ __forceinline__ void mma_split3(f32x4_t (&acc)[NB], const Split3& a, 
 // One 32-wide fp32 slab from the split terms.
 template <class G, int MBE>
 __device__ __forceinline__ void slab_mma_split3(f32x4_t (&acc)[MBE][G::NB], const uint16_t* sA, const uint16_t* sB,
-                                                int wm, int wn, int lane) {
+                                                int wm, int wn, int lane, uint32_t& lost) {
   const int lr = lane & 15;
   const int q = lane >> 4;
   Split3 b[G::NB];
 #pragma unroll
-  for (int j = 0; j < G::NB; ++j) b[j] = split3_lds(sB, wn * G::WN + j * 16 + lr, q);
+  for (int j = 0; j < G::NB; ++j) b[j] = split3_lds(sB, wn * G::WN + j * 16 + lr, q, lost);
 #pragma unroll
-  for (int i = 0; i < MBE; ++i) mma_split3<G::NB>(acc[i], split3_lds(sA, wm * 16 * MBE + i * 16 + lr, q), b);
+  for (int i = 0; i < MBE; ++i) mma_split3<G::NB>(acc[i], split3_lds(sA, wm * 16 * MBE + i * 16 + lr, q, lost), b);
 }
 
-// Whether the split terms may not stand for a tile's operands, told from its sums: one is infinite or
-// NaN, or nonzero below 2^-64 (operands below 2^-109 reach past the smallest bf16, 2^-133, before their
-// 24 bits end; ordinary sums that small are cancellations of about one in 10^18).
+// Whether the split terms may not stand for a tile's operands: one of them does not fit its three terms, or
+// a sum is infinite or NaN (an operand that is, or a product past the fp32 range).
 template <class G, int MBE>
-__device__ __forceinline__ bool split3_doubtful(const f32x4_t (&acc)[MBE][G::NB]) {
-  bool bad = false;
+__device__ __forceinline__ bool split3_doubtful(const f32x4_t (&acc)[MBE][G::NB], uint32_t lost) {
+  bool bad = (lost & 0xffffu) != 0;
 #pragma unroll
   for (int i = 0; i < MBE; ++i)
 #pragma unroll
     for (int j = 0; j < G::NB; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float m = fabsf(acc[i][j][r]);
-        bad |= !(m <= 3.4028234663852886e38f) | ((m < 0x1p-64f) & (m != 0.f));
-      }
+      for (int r = 0; r < 4; ++r) bad |= !(fabsf(acc[i][j][r]) <= 3.4028234663852886e38f);
   return bad;
 }
 
@@ -390,9 +397,9 @@ constexpr int kSplit3MinRows = 32;
 // of the split terms.
 template <class G, int MBE, int OPS = kSlabBF16>
 __device__ __forceinline__ void slab_mma(f32x4_t (&acc)[MBE][G::NB], const uint16_t* sA, const uint16_t* sB, int wm,
-                                         int wn, int lane) {
+                                         int wn, int lane, uint32_t& lost) {
   if constexpr (OPS == kSlabSplit3) {
-    slab_mma_split3<G, MBE>(acc, sA, sB, wm, wn, lane);
+    slab_mma_split3<G, MBE>(acc, sA, sB, wm, wn, lane, lost);
   } else {
 #pragma unroll
     for (int kk = 0; kk < G::BK / 32; ++kk) {
@@ -705,7 +712,8 @@ __device__ __forceinline__ void a_offsets(const GemmArgs& p, const TileCoord& tc
 // F32: fp32 A and B.  An LDS row is 128 bytes either way (64 bf16 or 32 fp32 of K per slab), so
 // the DMA, the swizzle and the fragment reads are the same bytes; only the MFMA differs.
 template <int BM, int BN, int WGM, int WGN, int EPI, int GM, bool F32 = false>
-__global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_dma_kernel(GemmArgs p) {
+__global__ void __launch_bounds__(WGM * WGN * 64, F32 && BM >= kSplit3MinRows ? (BM == 128 ? 2 : 3) : 1)
+grouped_gemm_dma_kernel(GemmArgs p) {
   using G = Geo<BM, BN, WGM, WGN, EPI>;
   constexpr int EB = F32 ? 4 : 2;             // bytes per element
   constexpr int BK = G::BK;
@@ -755,6 +763,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_dma_kernel(GemmAr
   by_height<BM, G::MB, A_PW>(tc.row_end - tc.row0, [&]<int MBE>() {
     constexpr int A_CNT = A_PW * MBE / G::MB;
     f32x4_t acc[MBE][G::NB];
+    uint32_t lost = 0;
     auto k_loop = [&]<int OPS>() {
 #pragma unroll
       for (int i = 0; i < MBE; ++i)
@@ -770,22 +779,22 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_dma_kernel(GemmAr
       for (; kt + 1 < KT; kt += 2) {
         issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA1, sB1, wave, (kt + 1) * BK * 2, b_nt);
         pin_issue();
-        slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane);
+        slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane, lost);
         __syncthreads();
         issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, min(kt + 2, KT - 1) * BK * 2,
                                         b_nt);
         pin_issue();
-        slab_mma<G, MBE, OPS>(acc, sA1, sB1, wm, wn, lane);
+        slab_mma<G, MBE, OPS>(acc, sA1, sB1, wm, wn, lane, lost);
         __syncthreads();
       }
-      if (kt < KT) slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane);   // odd slab count: last slab in buffer 0
+      if (kt < KT) slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane, lost);   // odd slab count: last slab in buffer 0
     };
     if constexpr (F32 && BM >= kSplit3MinRows) {
-      // Infinite and NaN operands (and products past the fp32 range) leave sums that are not finite,
-      // as on the fp32 MFMA but not the same ones (inf * 0 among the split terms): such a tile is
-      // computed again on the fp32 MFMA.  The vote is also the barrier before the stages are reused.
+      // Operands that do not fit their three terms lose bits; infinite and NaN operands (and products past
+      // the fp32 range) leave sums that are not finite, as on the fp32 MFMA but not the same ones (inf * 0
+      // among the split terms).  Such a tile is computed again on the fp32 MFMA.  The vote is also the barrier before the stages are reused.
       k_loop.template operator()<kSlabSplit3>();
-      if (__syncthreads_or(split3_doubtful<G, MBE>(acc) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
+      if (__syncthreads_or(split3_doubtful<G, MBE>(acc, lost) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
     } else {
       k_loop.template operator()<F32 ? kSlabF32 : kSlabBF16>();
     }
@@ -945,11 +954,12 @@ __device__ __forceinline__ void ring_frag_addrs(uint32_t aA, uint32_t aB, int wm
 // A slab's MFMAs from its fragments (both K halves: A then B of half 0, then of half 1).  For fp32 the
 // halves are the chunks q and q + 4 of each row, which the split takes as one 32-wide fragment.
 template <class G, int MBE, int OPS>
-__device__ __forceinline__ void ring_mma(f32x4_t (&acc)[MBE][G::NB], bf16x8_t (&fr)[2 * (MBE + G::NB)]) {
+__device__ __forceinline__ void ring_mma(f32x4_t (&acc)[MBE][G::NB], bf16x8_t (&fr)[2 * (MBE + G::NB)],
+                                         uint32_t& lost) {
   constexpr int F = MBE + G::NB;
   if constexpr (OPS == kSlabSplit3) {
     auto split = [&](int i) {
-      return split3(__builtin_bit_cast(f32x4_t, fr[i]), __builtin_bit_cast(f32x4_t, fr[F + i]));
+      return split3(__builtin_bit_cast(f32x4_t, fr[i]), __builtin_bit_cast(f32x4_t, fr[F + i]), lost);
     };
     Split3 b[G::NB];
 #pragma unroll
@@ -1025,6 +1035,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     // wave finished reading it before the barrier that ended that slab).
     // The slab's DMA goes first, then its fragment reads and their wait (lds_read_wait), its MFMAs, and
     // the wait for the next slab's data.
+    uint32_t lost = 0;
     auto k_loop = [&]<int OPS>() {
 #pragma unroll
       for (int i = 0; i < MBE; ++i)
@@ -1043,7 +1054,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     ring_frag_addrs<G, MBE>(lds_addr(SA), lds_addr(SB), wm, wn, lane, ad);                                  \
     bf16x8_t fr[2 * (MBE + G::NB)];                                                                         \
     lds_read_wait(ad, fr);                                                                                  \
-    ring_mma<G, MBE, OPS>(acc, fr);                                                                         \
+    ring_mma<G, MBE, OPS>(acc, fr, lost);                                                                   \
     wait_vm<(NS - 2) * L>();                                                                                \
     pp_barrier();                                                                                           \
   }
@@ -1057,7 +1068,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     };
     if constexpr (F32 && BM >= kSplit3MinRows) {
       k_loop.template operator()<kSlabSplit3>();   // as in grouped_gemm_dma_kernel
-      if (__syncthreads_or(split3_doubtful<G, MBE>(acc) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
+      if (__syncthreads_or(split3_doubtful<G, MBE>(acc, lost) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
     } else {
       k_loop.template operator()<F32 ? kSlabF32 : kSlabBF16>();
     }

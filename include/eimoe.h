@@ -55,7 +55,11 @@ enum {
   EIMOE_FP32 = 32        /* fp32 layer: x, the weights (w_dtype EIMOE_F32, shared weights too), h
                             and y in fp32, products to fp32's error (the reference's fp32 F.linear
                             path, native_moe.py:56-103).  Required with, and only with, fp32 weights;
-                            size the workspace with it.  Not with W8A8 or H_SPLIT. */
+                            size the workspace with it.  Not with W8A8 or H_SPLIT.  Tiles of 32 rows and
+                            more multiply three bf16 terms of each operand; a tile with an operand
+                            that these do not hold (its bits end below 2^-133), an infinity or NaN is
+                            computed with fp32 products, so that the last bits of a row may depend on
+                            the other rows of its expert. */
 };
 
 /* tile selector for the GEMM entry points (0 = automatic).  EIMOE_TILE_STREAM is the

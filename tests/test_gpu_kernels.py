@@ -1038,8 +1038,8 @@ def test_ring_lds_tiles_bit_identical_with_two_stage(dev, tile, bm, bn, mode):
         assert torch.equal(dn(rows, ks), dn(bounds[f"dn{ks}"], ks))
 
 
-# The fp32 tiles of 32 rows and more multiply three bf16 terms per operand on the bf16 MFMA; a tile whose
-# sums are not finite, or nonzero below 2^-64, is computed again on the fp32 MFMA.  Every tile, on the
+# The fp32 tiles of 32 rows and more multiply three bf16 terms per operand on the bf16 MFMA; a tile with an
+# operand that the terms do not hold, or with sums that are not finite, is computed again on the fp32 MFMA.  Every tile, on the
 # two-stage kernel and on the ring (row bounds in both regimes), against float64: ordinary values,
 # infinities, NaN, zero rows and the largest finite values, and operands near the smallest normal.
 # Bound: K rounded additions of partial sums below the norm n of the products, of rms 2^-24 n sqrt(K/2)
@@ -1084,3 +1084,30 @@ def test_fp32_split_terms(dev, tile, counts, values):
         norm = ((x[:, None, :] * w[None, :, :]) ** 2).sum(-1).sqrt()
         err = (got - ref).abs()
         assert (err[fin] <= 6 * math.sqrt(K / 2) * 2.0 ** -24 * norm[fin]).all()
+
+
+# Operands whose last bits lie below the smallest bf16 (2^-133), times large ones so that the sums are
+# ordinary: all of them, or one row or weight row among ordinary values, which sit in the same tile.  Same
+# bound as above; the fp32 MFMA multiplies subnormal operands as they are.
+@pytest.mark.parametrize("tile", [2, 3, 6])
+@pytest.mark.parametrize("counts", [[33, 0, 70, 1], [400, 129, 700, 260]])
+@pytest.mark.parametrize("ea,eb,only", [(-118, 100, None), (-122, 90, None), (-125, 80, None), (-140, 90, None),
+                                        (90, -140, None), (-125, 80, "row"), (-140, 40, "row"), (80, -125, "weight")])
+def test_fp32_small_operands_keep_their_bits(dev, tile, counts, ea, eb, only):
+    g = torch.Generator().manual_seed(7 + tile)
+    E, N, K = len(counts), 256, 320
+    off, off_t = _segments(counts)
+    rows = int(off[-1])
+    a = torch.randn(rows, K, generator=g)
+    b = torch.randn(E, N, K, generator=g)
+    sa, sb = torch.ones(rows, 1), torch.ones(E, N, 1)
+    sa[[5, rows - 1] if only == "row" else slice(None)] = 2.0 ** ea
+    sb[:, [17, 200] if only == "weight" else slice(None)] = 2.0 ** eb
+    a, b = a * sa, b * sb
+    c = cpu(ops.grouped_gemm(a.to(dev), b.to(dev), off_t.to(dev), rows, out_dtype=torch.float32, tile=tile))
+    for e in range(E):
+        lo, hi = int(off[e]), int(off[e + 1])
+        x, w = a[lo:hi].double(), b[e].double()
+        norm = (x ** 2 @ (w ** 2).T).sqrt()
+        err = (c[lo:hi].double() - x @ w.T).abs()
+        assert (err <= 6 * math.sqrt(K / 2) * 2.0 ** -24 * norm).all()
