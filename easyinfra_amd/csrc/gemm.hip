@@ -307,17 +307,21 @@ __device__ __forceinline__ void mma_f32(f32x4_t (&acc)[MBE][G::NB], const bf16x8
   }
 }
 
+// What a slab's MFMAs take: bf16 operands, fp32 operands on the fp32 MFMA, fp32 operands split.
+enum SlabOps : int { kSlabBF16 = 0, kSlabF32 = 1, kSlabSplit3 = 2 };
+
 // a |= b | c, in one instruction and where it stands: the compiler would gather a slab's into one tree and
 // keep all their operands (up to 64 registers a lane) until then.
 __device__ __forceinline__ void or3(uint32_t& a, uint32_t b, uint32_t c) {
   asm("v_or3_b32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
 }
 
-// fp32 operands as three bf16 terms on the bf16 MFMA: x = hi + mid + lo, each the upper half of what
-// the terms before it leave.  A fp32 mantissa has 24 bits and each term takes 8, so the three hold x
-// exactly while lo stays above the smallest bf16 (2^-133: operands down to 2^-109, and smaller ones whose
-// bits end in time).  `lost` collects what does not fit, in its lower half.  Lane group q's eight values of
-// a 32-wide k slab are the 16-byte chunks q and q + 4 of the row, for A and B alike.
+// fp32 operands as three bf16 terms on the bf16 MFMA: x = hi + mid + lo, hi and mid each what the terms
+// before it leave, rounded to bf16, lo the rest.  A fp32 mantissa has 24 bits and each term takes 8, so the
+// three hold x exactly while lo stays above the smallest bf16 (2^-133; operands down to 2^-109 and the
+// smaller ones whose bits end in time); `lost` collects what does not fit, the low halves of lo.
+// Lane group q's eight values of a 32-wide k slab are the 16-byte chunks q and q + 4 of the row, for A and
+// B alike.
 struct Split3 {
   bf16x8_t t[3];   // hi, mid, lo
 };
@@ -329,16 +333,14 @@ __device__ __forceinline__ Split3 split3(const f32x4_t& c0, const f32x4_t& c1, u
     float x0 = i < 2 ? c0[2 * i] : c1[2 * i - 4];
     float x1 = i < 2 ? c0[2 * i + 1] : c1[2 * i - 3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
-      w[k][i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);   // the upper halves
-      if (k == 2) {
-        or3(lost, u0, u1);
-        break;
-      }
-      x0 -= __uint_as_float(u0 & 0xffff0000u);
-      x1 -= __uint_as_float(u1 & 0xffff0000u);
+    for (int k = 0; k < 2; ++k) {
+      w[k][i] = pack_bf16x2(x0, x1);
+      x0 -= __uint_as_float(w[k][i] << 16);
+      x1 -= __uint_as_float(w[k][i] & 0xffff0000u);
     }
+    const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+    w[2][i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);   // the upper halves
+    or3(lost, u0, u1);
   }
   return Split3{{__builtin_bit_cast(bf16x8_t, w[0]), __builtin_bit_cast(bf16x8_t, w[1]),
                  __builtin_bit_cast(bf16x8_t, w[2])}};
@@ -349,16 +351,44 @@ __device__ __forceinline__ Split3 split3_lds(const uint16_t* s, int R, int q, ui
                 *reinterpret_cast<const f32x4_t*>(&s[R * 64 + (((q + 4) ^ swz(R)) << 3)]), lost);
 }
 
-// One row of fragments times all columns: the six products above 2^-22 of x*y, smallest first.
-template <int NB>
-__device__ __forceinline__ void mma_split3(f32x4_t (&acc)[NB], const Split3& a, const Split3 (&b)[NB]) {
+// One column of fragments times all rows: six of the nine products, smallest first.  The three left out
+// are at most 2^-24 of x*y together, of either sign.  (Column by column: the terms of one weight fragment
+// are live at a time, so that the chain fits beside the sums at three waves a SIMD on 64x128.)
+template <int MBE, int NB>
+__device__ __forceinline__ void mma_split3(f32x4_t (&acc)[MBE][NB], int j, const Split3 (&a)[MBE], const Split3& b) {
   constexpr int ta[6] = {2, 0, 1, 1, 0, 0};
   constexpr int tb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
   for (int k = 0; k < 6; ++k)
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.t[ta[k]], b[j].t[tb[k]], acc[j], 0, 0, 0);
+    for (int i = 0; i < MBE; ++i)
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i].t[ta[k]], b.t[tb[k]], acc[i][j], 0, 0, 0);
+}
+
+// The bf16 MFMA drops what its products have below the accumulator's last bits, which adds up where the
+// operands have one sign: in one chain over K = 2816 the error of |N(0, 1)| operands against float64 was
+// 5.6e-6 (fp32 MFMA 7.4e-7).  So a chain ends after kSplit3Chain slabs and is added to the tile's sums by
+// v_add_f32: 7.0e-8, on N(0, 1) operands 2.1e-7 (fp32 MFMA 9.5e-7).  A multiple of both kernels' slabs per
+// iteration (two, three), so that they add alike.
+constexpr int kSplit3Chain = 6;
+
+template <int MBE, int NB>
+__device__ __forceinline__ void split3_add_chain(f32x4_t (&acc)[MBE][NB], f32x4_t (&chain)[MBE][NB]) {
+#pragma unroll
+  for (int i = 0; i < MBE; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] += chain[i][j][r];
+      chain[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+// What a slab's MFMAs add to: a chain of its own for the split terms, else the tile's sums.
+template <int OPS, int MBE, int NB>
+__device__ __forceinline__ f32x4_t (&slab_acc(f32x4_t (&acc)[MBE][NB], f32x4_t (&chain)[MBE][NB]))[MBE][NB] {
+  if constexpr (OPS == kSlabSplit3) return chain;
+  else return acc;
 }
 
 // One 32-wide fp32 slab from the split terms.
@@ -367,15 +397,15 @@ __device__ __forceinline__ void slab_mma_split3(f32x4_t (&acc)[MBE][G::NB], cons
                                                 int wm, int wn, int lane, uint32_t& lost) {
   const int lr = lane & 15;
   const int q = lane >> 4;
-  Split3 b[G::NB];
+  Split3 a[MBE];
 #pragma unroll
-  for (int j = 0; j < G::NB; ++j) b[j] = split3_lds(sB, wn * G::WN + j * 16 + lr, q, lost);
+  for (int i = 0; i < MBE; ++i) a[i] = split3_lds(sA, wm * 16 * MBE + i * 16 + lr, q, lost);
 #pragma unroll
-  for (int i = 0; i < MBE; ++i) mma_split3<G::NB>(acc[i], split3_lds(sA, wm * 16 * MBE + i * 16 + lr, q, lost), b);
+  for (int j = 0; j < G::NB; ++j) mma_split3<MBE, G::NB>(acc, j, a, split3_lds(sB, wn * G::WN + j * 16 + lr, q, lost));
 }
 
 // Whether the split terms may not stand for a tile's operands: one of them does not fit its three terms, or
-// a sum is infinite or NaN (an operand that is, or a product past the fp32 range).
+// a sum is infinite or NaN (an operand that is, or one that rounds to an infinite hi).
 template <class G, int MBE>
 __device__ __forceinline__ bool split3_doubtful(const f32x4_t (&acc)[MBE][G::NB], uint32_t lost) {
   bool bad = (lost & 0xffffu) != 0;
@@ -388,8 +418,6 @@ __device__ __forceinline__ bool split3_doubtful(const f32x4_t (&acc)[MBE][G::NB]
   return bad;
 }
 
-// What a slab's MFMAs take: bf16 operands, fp32 operands on the fp32 MFMA, fp32 operands split.
-enum SlabOps : int { kSlabBF16 = 0, kSlabF32 = 1, kSlabSplit3 = 2 };
 // fp32 tiles of at least this many rows take the split terms; below, the fp32 MFMA.
 constexpr int kSplit3MinRows = 32;
 
@@ -765,10 +793,12 @@ grouped_gemm_dma_kernel(GemmArgs p) {
     f32x4_t acc[MBE][G::NB];
     uint32_t lost = 0;
     auto k_loop = [&]<int OPS>() {
+      f32x4_t chain[MBE][G::NB];
 #pragma unroll
       for (int i = 0; i < MBE; ++i)
 #pragma unroll
-        for (int j = 0; j < G::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < G::NB; ++j) acc[i][j] = chain[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      auto& to = slab_acc<OPS>(acc, chain);
       issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, 0, b_nt);
       __syncthreads();
       int kt = 0;
@@ -776,18 +806,29 @@ grouped_gemm_dma_kernel(GemmArgs p) {
       // (on the last iteration of an even slab count it re-reads slab KT-1 into buffer 0, which is
       // not read again and which the closing barrier waits for) so that it is not split into its
       // own basic block, where the scheduler would queue the previous slab's MFMAs ahead of it.
-      for (; kt + 1 < KT; kt += 2) {
-        issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA1, sB1, wave, (kt + 1) * BK * 2, b_nt);
-        pin_issue();
-        slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane, lost);
-        __syncthreads();
-        issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, min(kt + 2, KT - 1) * BK * 2,
-                                        b_nt);
-        pin_issue();
-        slab_mma<G, MBE, OPS>(acc, sA1, sB1, wm, wn, lane, lost);
-        __syncthreads();
+      auto pairs = [&](int stop) {
+        for (; kt + 1 < stop; kt += 2) {
+          issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA1, sB1, wave, (kt + 1) * BK * 2, b_nt);
+          pin_issue();
+          slab_mma<G, MBE, OPS>(to, sA0, sB0, wm, wn, lane, lost);
+          __syncthreads();
+          issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, sA0, sB0, wave, min(kt + 2, KT - 1) * BK * 2,
+                                          b_nt);
+          pin_issue();
+          slab_mma<G, MBE, OPS>(to, sA1, sB1, wm, wn, lane, lost);
+          __syncthreads();
+        }
+      };
+      if constexpr (OPS == kSlabSplit3) {
+        while (kt + 1 < KT) {
+          pairs(min(kt + kSplit3Chain, KT));
+          if (kt % kSplit3Chain == 0) split3_add_chain(acc, chain);
+        }
+      } else {
+        pairs(KT);
       }
-      if (kt < KT) slab_mma<G, MBE, OPS>(acc, sA0, sB0, wm, wn, lane, lost);   // odd slab count: last slab in buffer 0
+      if (kt < KT) slab_mma<G, MBE, OPS>(to, sA0, sB0, wm, wn, lane, lost);   // odd slab count: last slab in buffer 0
+      if constexpr (OPS == kSlabSplit3) split3_add_chain(acc, chain);
     };
     if constexpr (F32 && BM >= kSplit3MinRows) {
       // Operands that do not fit their three terms lose bits; infinite and NaN operands (and products past
@@ -961,11 +1002,11 @@ __device__ __forceinline__ void ring_mma(f32x4_t (&acc)[MBE][G::NB], bf16x8_t (&
     auto split = [&](int i) {
       return split3(__builtin_bit_cast(f32x4_t, fr[i]), __builtin_bit_cast(f32x4_t, fr[F + i]), lost);
     };
-    Split3 b[G::NB];
+    Split3 a[MBE];
 #pragma unroll
-    for (int j = 0; j < G::NB; ++j) b[j] = split(MBE + j);
+    for (int i = 0; i < MBE; ++i) a[i] = split(i);
 #pragma unroll
-    for (int i = 0; i < MBE; ++i) mma_split3<G::NB>(acc[i], split(i), b);
+    for (int j = 0; j < G::NB; ++j) mma_split3<MBE, G::NB>(acc, j, a, split(MBE + j));
   } else {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
@@ -1037,10 +1078,12 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     // the wait for the next slab's data.
     uint32_t lost = 0;
     auto k_loop = [&]<int OPS>() {
+      f32x4_t chain[MBE][G::NB];
 #pragma unroll
       for (int i = 0; i < MBE; ++i)
 #pragma unroll
-        for (int j = 0; j < G::NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < G::NB; ++j) acc[i][j] = chain[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      auto& to = slab_acc<OPS>(acc, chain);
       // slabs 0 and 1 into stages 0 and 1 (clamped to the last slab: stages not read again)
       issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, t0.a, t0.b, wave, 0, b_nt);
       issue_slab_dma<A_CNT, B_PW, NW>(rA, rB, a_voff, b_voff, t1.a, t1.b, wave, min(1, KT - 1) * BK * 2, b_nt);
@@ -1054,7 +1097,7 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
     ring_frag_addrs<G, MBE>(lds_addr(SA), lds_addr(SB), wm, wn, lane, ad);                                  \
     bf16x8_t fr[2 * (MBE + G::NB)];                                                                         \
     lds_read_wait(ad, fr);                                                                                  \
-    ring_mma<G, MBE, OPS>(acc, fr, lost);                                                                   \
+    ring_mma<G, MBE, OPS>(to, fr, lost);                                                                    \
     wait_vm<(NS - 2) * L>();                                                                                \
     pp_barrier();                                                                                           \
   }
@@ -1062,8 +1105,11 @@ __global__ void __launch_bounds__(WGM * WGN * 64) grouped_gemm_ring_kernel(GemmA
         EIMOE_RING_SLAB(0, t0.a, t0.b, t2.a, t2.b)
         EIMOE_RING_SLAB(1, t1.a, t1.b, t0.a, t0.b)
         EIMOE_RING_SLAB(2, t2.a, t2.b, t1.a, t1.b)
+        if constexpr (OPS == kSlabSplit3)
+          if (kt % kSplit3Chain == kSplit3Chain - NS) split3_add_chain(acc, chain);
       }
 #undef EIMOE_RING_SLAB
+      if constexpr (OPS == kSlabSplit3) split3_add_chain(acc, chain);
       pp_wait_vm0();   // the clamped loads near the end land before the workgroup's LDS is released (or reused)
     };
     if constexpr (F32 && BM >= kSplit3MinRows) {
@@ -2552,7 +2598,7 @@ static hipError_t launch_cfg_f32(const GemmArgs& p, int max_rows, hipStream_t s)
   // The ring where its workgroups hold all the expected tiles in one round (weights streamed at a few
   // rows per expert: the tiny-Mixtral gate/up at 2 / 8 / 24 rows in all 27.3 / 30.0 / 35.5 -> 18.2 / 23.3 /
   // 34.1 us on 16x64, its down projection with K split 4 20.0 / 20.9 / 23.2 -> 13.6 / 14.6 / 18.8); past
-  // one round the two-stage kernel's extra workgroups per CU win (512 rows on 64x128: 75.4 against 87.2).
+  // one round the two-stage kernel's extra workgroups per CU win (512 rows on 64x128: 85 against 90).
   if constexpr (BM <= 64) {
     const int S = p.S > 0 ? p.S : 1;
     const double avg = static_cast<double>(p.rows_hint > 0 ? std::min(p.rows_hint, p.max_rows) : p.max_rows) / S;
@@ -2582,12 +2628,12 @@ static hipError_t launch_epi_f32(const GemmArgs& p, int max_rows, int tile, hipS
 // fp32 tiles.  16x64 multiplies on the fp32 MFMA (its few rows are bound by the weights), the taller
 // tiles split their operands into bf16 terms: six bf16 MFMAs cost 6/16 of the fp32 one.  By expected
 // rows per segment, measured on the tiny-Mixtral shape (8 experts, 1024 x 2816, cold, one box; us):
-// gate/up on 16x64 / 32x128 / 64x128 / 128x128 at 16 rows 37 / 40 / 40 / 50, at 24 rows 44 / 39 / 50 /
-// 54, at 32 rows 67 / 52 / 52 / 62, at 96 rows 123 / 98 / 80 / 84, at 128 rows 167 / 124 / 103 / 135, at
-// 256 rows 366 / 217 / 168 / 165, at 512 rows 776 / 407 / 298 / 295; down (K split 4) at 16 rows 20 / 21 /
-// 23 / 29, at 32 rows 27 / 26 / 29 / 33, at 64 rows 44 / 39 / 40 / 46, at 128 rows 68 / 60 / 55 / 62, at 256
-// rows 123 / 100 / 87 / 103.  The layer at 512 tokens: 251 -> 175 us against the fp32 MFMA on
-// 128x128, error against float64 9.9e-7 -> 8.7e-7; at 1 / 40 tokens 56 -> 44 / 68 -> 61 us.
+// gate/up on 16x64 / 32x128 / 64x128 / 128x128 at 16 rows 40 / 46 / 48 / 47, at 24 rows 46 / 46 / 49 /
+// 47, at 32 rows 69 / 49 / 60 / 59, at 96 rows 128 / 98 / 89 / 97, at 128 rows 184 / 131 / 113 / 141, at
+// 256 rows 380 / 221 / 187 / 181, at 512 rows 782 / 416 / 318 / 309; down (K split 4) at 16 rows 21 / 22 /
+// 24 / 29, at 32 rows 26 / 31 / 30 / 31, at 64 rows 43 / 41 / 45 / 46, at 128 rows 69 / 65 / 61 / 66, at 256
+// rows 122 / 110 / 96 / 112.  Layers against the fp32 MFMA on 128x128: 512 tokens 289 -> 194 us, error
+// against float64 9.9e-7 -> 3.7e-7; 1 / 40 / 2048 tokens 53 -> 38 / 72 -> 62 / 688 -> 513 us.
 hipError_t launch_grouped_gemm_f32(const GemmArgs& p, int epi, int max_rows, int tile, hipStream_t s) {
   if (epi != kEpiSiluF32 && epi != kEpiStoreF32) return hipErrorInvalidValue;
   if (tile == kTileAuto) {

@@ -1043,7 +1043,7 @@ def test_ring_lds_tiles_bit_identical_with_two_stage(dev, tile, bm, bn, mode):
 # two-stage kernel and on the ring (row bounds in both regimes), against float64: ordinary values,
 # infinities, NaN, zero rows and the largest finite values, and operands near the smallest normal.
 # Bound: K rounded additions of partial sums below the norm n of the products, of rms 2^-24 n sqrt(K/2)
-# when taken as independent, six times that; the products left out are below 2^-22 each.  (A missing
+# when taken as independent, six times that; the products left out are below 2^-24 each.  (A missing
 # term, or one cut at the smallest bf16, is 2^-16 n, three times the bound.)
 @pytest.mark.parametrize("tile", [2, 3, 6])
 @pytest.mark.parametrize("counts", [[33, 0, 70, 1], [400, 129, 700, 260]])
@@ -1111,3 +1111,21 @@ def test_fp32_small_operands_keep_their_bits(dev, tile, counts, ea, eb, only):
         norm = (x ** 2 @ (w ** 2).T).sqrt()
         err = (c[lo:hi].double() - x @ w.T).abs()
         assert (err <= 6 * math.sqrt(K / 2) * 2.0 ** -24 * norm).all()
+
+
+# Operands of one sign, where what each addition drops adds up instead of averaging, and one repeated value
+# whose terms are all at their largest (1 + 2^-7 - 2^-23).  Bound: the rms of a sum of K products in K / 4
+# rounded additions, as the fp32 MFMA adds them, each off by at most half a unit of a partial sum that grows
+# evenly: 2^-24 sqrt(K / 12).
+@pytest.mark.parametrize("tile", [2, 3, 6])
+@pytest.mark.parametrize("values,K", [("normal", 2816), ("uniform", 2816), ("uniform", 14336), ("repeated", 64)])
+def test_fp32_sums_of_one_sign(dev, tile, values, K):
+    g = torch.Generator().manual_seed(K)
+    rows, N = 129, 256
+    draw = {"normal": lambda *s: torch.randn(*s, generator=g).abs(), "uniform": lambda *s: torch.rand(*s, generator=g),
+            "repeated": lambda *s: torch.full(s, 1 + 2.0 ** -7 - 2.0 ** -23)}[values]
+    a, b = draw(rows, K), draw(1, N, K)
+    off = torch.tensor([0, rows], dtype=torch.int32)
+    c = cpu(ops.grouped_gemm(a.to(dev), b.to(dev), off.to(dev), rows, out_dtype=torch.float32, tile=tile)).double()
+    ref = a.double() @ b[0].double().T
+    assert float((c - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(K / 12)
