@@ -226,8 +226,9 @@ hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offse
 // expert is one segment.  offsets[n_exp + 1]: the experts' bounds in merged order; rows[m]: the
 // original row of merged row m; pos[r]: the merged row of original row r, -1 for rows past the last
 // segment.  Only integers, one launch (it stands in for counts_to_offsets, ~4.5 us either way).
-// Segment bounds are clamped to [0, max_rows] and made monotonic as the GEMM does, so that every
-// merged row below offsets[n_exp] names a row below max_rows whatever the counts say.
+// A negative count stands for an empty segment and the bounds end at max_rows, so that segments never
+// overlap: every entry of pos is written, and every merged row below offsets[n_exp] names a row below
+// max_rows, whatever the counts say.
 // Workgroup s copies segment s's run; each recomputes the prefix sums of the (at most 1024) counts.
 __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __restrict__ counts, int S, int n_exp,
                                                              int max_rows, int32_t* __restrict__ offsets,
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
   static_assert(256 * kPer >= kMaxSeg, "one pass over the segments");
   __shared__ int s_wave[4];
   __shared__ int s_bound[256 * kPer + 1];
-  __shared__ int s_red[4][3];
+  __shared__ int s_red[4];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wv = tid >> 6;
@@ -246,56 +247,43 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     const int s = tid * kPer + j;
-    c[j] = s < S ? counts[s] : 0;
-    sum += c[j];
+    c[j] = s < S ? min(max(counts[s], 0), max_rows) : 0;
+    sum = min(sum + c[j], max_rows);
   }
+  // Sums past max_rows stay there: with at most 2^24 rows (2 GiB of 64 columns) nothing leaves 32 bits.
   const int incl = wave_incl_scan(sum);
-  if (lane == 63) s_wave[wv] = incl;
+  if (lane == 63) s_wave[wv] = min(incl, max_rows);
   __syncthreads();
   int run = incl - sum;
   for (int w = 0; w < wv; ++w) run += s_wave[w];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    s_bound[tid * kPer + j] = run;
+    s_bound[tid * kPer + j] = min(run, max_rows);
     run += c[j];
   }
-  if (tid == 255) s_bound[256 * kPer] = run;
+  if (tid == 255) s_bound[256 * kPer] = min(run, max_rows);
   __syncthreads();
-  // rows of segment s after clamping; of this thread's segments: those before `seg` in merged order
-  // (a lower expert, or the same expert of a lower rank), and all
+  // of this thread's segments, the rows of those before `seg` in merged order (a lower expert, or the same
+  // expert of a lower rank)
   const int e = seg % n_exp;
-  int before = 0, all = 0, last = 0;
+  int before = 0;
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     const int s = tid * kPer + j;
     if (s >= S) continue;
-    const int r0 = min(max(s_bound[s], 0), max_rows);
-    const int r1 = min(max(s_bound[s + 1], r0), max_rows);
     const int es = s % n_exp;
-    if (es < e || (es == e && s < seg)) before += r1 - r0;
-    all += r1 - r0;
-    last = max(last, r1);
+    if (es < e || (es == e && s < seg)) before += s_bound[s + 1] - s_bound[s];
   }
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    before += __shfl_xor(before, m, 64);
-    all += __shfl_xor(all, m, 64);
-    last = max(last, __shfl_xor(last, m, 64));
-  }
-  if (lane == 0) {
-    s_red[wv][0] = before;
-    s_red[wv][1] = all;
-    s_red[wv][2] = last;
-  }
+  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
+  if (lane == 0) s_red[wv] = before;
   __syncthreads();
-  const int dst = min(s_red[0][0] + s_red[1][0] + s_red[2][0] + s_red[3][0], max_rows);
-  const int total = min(s_red[0][1] + s_red[1][1] + s_red[2][1] + s_red[3][1], max_rows);
-  const int end = max(max(s_red[0][2], s_red[1][2]), max(s_red[2][2], s_red[3][2]));
-  const int r0 = min(max(s_bound[seg], 0), max_rows);
-  const int r1 = min(max(s_bound[seg + 1], r0), max_rows);
-  const int n = min(r1 - r0, max_rows - dst);
+  const int dst = s_red[0] + s_red[1] + s_red[2] + s_red[3];
+  const int end = s_bound[S];
+  const int r0 = s_bound[seg];
+  const int n = s_bound[seg + 1] - r0;
   if (tid == 0 && seg < n_exp) offsets[seg] = dst;   // rank 0's segments start the experts
-  if (tid == 0 && seg == 0) offsets[n_exp] = total;
+  if (tid == 0 && seg == 0) offsets[n_exp] = end;
   for (int i = tid; i < n; i += 256) {
     rows[dst + i] = r0 + i;
     pos[r0 + i] = dst + i;
@@ -305,7 +293,8 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
 
 hipError_t launch_merge_segments(const int32_t* counts, int S, int n_exp, int max_rows, int32_t* offsets,
                                  int32_t* rows, int32_t* pos, hipStream_t s) {
-  if (S < 1 || S > kMaxSeg || n_exp < 1 || S % n_exp != 0) return hipErrorInvalidValue;
+  if (S < 1 || S > kMaxSeg || n_exp < 1 || S % n_exp != 0 || max_rows > (1 << 24))
+    return hipErrorInvalidValue;
   hipLaunchKernelGGL(merge_segments_kernel, dim3(static_cast<unsigned>(S)), dim3(256), 0, s, counts, S, n_exp,
                      max_rows, offsets, rows, pos);
   return hipGetLastError();

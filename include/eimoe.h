@@ -191,7 +191,8 @@ int eimoe_gemm_down_w8a8(const void* hq, const float* h_scale, int I, const void
 /* The experts' MLP on pre-grouped rows: FusedMoE.forward_ep(hidden_states, expert_count)
  * (fused_moe.py:106-156), unweighted.  x [M, H] holds the rows of segment s = rank * n_local + e one
  * after the other, counts[s] each (device int32, n_seg a multiple of n_local); y [M, H_out] keeps
- * their order.  Rows of one expert from several source ranks are computed as one segment, so its
+ * their order.  A negative count is an empty segment, and rows past M are left out.  Rows of one
+ * expert from several source ranks are computed as one segment, so its
  * weights are read once.  w_gate_up [n_local, 2I, H], w_down [n_local, H_out, I]: bf16 or fp8 (with
  * channel scales) and x, y bf16; or all fp32.  h is rounded to bf16 (fp32 experts: fp32), y once from
  * the fp32 sums.  H, I, H_out multiples of 64.  workspace: eimoe_experts_workspace_bytes bytes. */

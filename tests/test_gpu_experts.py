@@ -136,3 +136,36 @@ def test_experts_tile_bounds(dev, E, H, I, rows, mode):
         r += c
     # one bf16 rounding of the output and of h, each at most 2^-9 of a value
     assert oracle.rel_l2(y.cpu().float(), ref.cpu()) <= 2.0 ** -8
+
+
+# Counts that come to more rows than x has, or that are negative (empty segments), on each route that
+# regroups the rows: straight to their places, fp32 planes, K split planes.
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,ep,H,I", [(4, 2, 128, 128), (2, 2, 1024, 16384), (1, 1, 1024, 16384)])
+@pytest.mark.parametrize("kind", ["over", "negative"])
+@pytest.mark.parametrize("mode", ["bf16", "fp32"])
+def test_experts_counts_off_the_rows(dev, E, ep, H, I, kind, mode):
+    M = 120
+    g = torch.Generator().manual_seed(E * ep)
+    S = E * ep
+    counts = torch.full((S,), {"over": 150 // S, "negative": 60 // S}[kind])
+    if kind == "over":
+        counts[0] = 2 ** 31 - 1 if S == 1 else counts[0]
+        counts[-1] = 2 ** 31 - 1
+    if kind == "negative":
+        counts[S // 2] = -10 if S > 2 else counts[S // 2]
+        counts[S - 1] = -(2 ** 31)
+    dt = torch.float32 if mode == "fp32" else torch.bfloat16
+    x = torch.randn(M, H, generator=g).to(dt)
+    wgu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(dt)
+    wd = (torch.randn(E, H, I, generator=g) * 0.05).to(dt)
+    print("CASE", dict(E=E, ep=ep, H=H, I=I, kind=kind, mode=mode), flush=True)
+    y = ops.experts(x.to(dev), wgu.to(dev), wd.to(dev), counts.to(torch.int32).to(dev), E)
+    ref, r = torch.zeros(M, H), 0
+    for s, c in enumerate(counts.tolist()):
+        n = min(max(c, 0), M - r)
+        ref[r:r + n] = oracle.expert_mlp(x[r:r + n].float(), wgu[s % E].float(), wd[s % E].float(),
+                                         round_h_bf16=mode != "fp32")
+        r += n
+    # the bounds of test_experts_match_oracle_per_segment
+    assert float((y.cpu().float() - ref)[:r].norm()) <= (2e-5 if mode == "fp32" else 2.0 ** -8) * float(ref.norm())
