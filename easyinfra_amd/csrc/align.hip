@@ -225,14 +225,17 @@ hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offse
 // reads each expert's weights once per rank and pads one tile per (rank, expert); merged, each
 // expert is one segment.  offsets[n_exp + 1]: the experts' bounds in merged order; rows[m]: the
 // original row of merged row m; pos[r]: the merged row of original row r, -1 for rows past the last
-// segment.  Only integers, one launch (it stands in for counts_to_offsets, ~4.5 us either way).
+// segment, of which tail (null: left as it is) gets tail_words words of zeros each.  One launch (it stands
+// in for counts_to_offsets, ~4.5 us either way).  One source rank (S = n_exp) whose rows need no map: rows
+// and pos null, one workgroup.
 // A negative count stands for an empty segment and the bounds end at max_rows, so that segments never
 // overlap: every entry of pos is written, and every merged row below offsets[n_exp] names a row below
 // max_rows, whatever the counts say.
 // Workgroup s copies segment s's run; each recomputes the prefix sums of the (at most 1024) counts.
 __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __restrict__ counts, int S, int n_exp,
                                                              int max_rows, int32_t* __restrict__ offsets,
-                                                             int32_t* __restrict__ rows, int32_t* __restrict__ pos) {
+                                                             int32_t* __restrict__ rows, int32_t* __restrict__ pos,
+                                                             uint32_t* __restrict__ tail, int tail_words) {
   constexpr int kPer = 4;   // segments per thread: 256 * 4 = kMaxSeg
   static_assert(256 * kPer >= kMaxSeg, "one pass over the segments");
   __shared__ int s_wave[4];
@@ -263,6 +266,14 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
   }
   if (tid == 255) s_bound[256 * kPer] = min(run, max_rows);
   __syncthreads();
+  const int end = s_bound[S];
+  if (tail)
+    for (int r = end + seg; r < max_rows; r += gridDim.x)
+      for (int i = tid; i < tail_words; i += 256) tail[static_cast<long long>(r) * tail_words + i] = 0u;
+  if (!rows) {
+    for (int s = tid; s <= S; s += 256) offsets[s] = s_bound[s];
+    return;
+  }
   // of this thread's segments, the rows of those before `seg` in merged order (a lower expert, or the same
   // expert of a lower rank)
   const int e = seg % n_exp;
@@ -279,7 +290,6 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
   if (lane == 0) s_red[wv] = before;
   __syncthreads();
   const int dst = s_red[0] + s_red[1] + s_red[2] + s_red[3];
-  const int end = s_bound[S];
   const int r0 = s_bound[seg];
   const int n = s_bound[seg + 1] - r0;
   if (tid == 0 && seg < n_exp) offsets[seg] = dst;   // rank 0's segments start the experts
@@ -292,11 +302,12 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
 }
 
 hipError_t launch_merge_segments(const int32_t* counts, int S, int n_exp, int max_rows, int32_t* offsets,
-                                 int32_t* rows, int32_t* pos, hipStream_t s) {
-  if (S < 1 || S > kMaxSeg || n_exp < 1 || S % n_exp != 0 || max_rows > (1 << 24))
+                                 int32_t* rows, int32_t* pos, void* tail, int tail_bytes, hipStream_t s) {
+  if (S < 1 || S > kMaxSeg || n_exp < 1 || S % n_exp != 0 || max_rows > (1 << 24) || !rows != !pos ||
+      (!rows && S != n_exp))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(merge_segments_kernel, dim3(static_cast<unsigned>(S)), dim3(256), 0, s, counts, S, n_exp,
-                     max_rows, offsets, rows, pos);
+  hipLaunchKernelGGL(merge_segments_kernel, dim3(rows ? static_cast<unsigned>(S) : 1u), dim3(256), 0, s, counts, S, n_exp,
+                     max_rows, offsets, rows, pos, static_cast<uint32_t*>(tail), tail_bytes / 4);
   return hipGetLastError();
 }
 

@@ -643,7 +643,7 @@ int grouped_gemm_impl(const void* a, const int32_t* a_rows, int a_nrows, int lda
   REQUIRE_PTR(c);
   if (b_dtype == EIMOE_FP8) REQUIRE_PTR(b_scale);
   if (merge && (rc = hip_check(launch_merge_segments(merge->counts, merge->n_seg, n_seg, max_rows, merge->offsets,
-                                                     merge->rows, merge->pos, S(stream)),
+                                                     merge->rows, merge->pos, nullptr, 0, S(stream)),
                                "merge segments")))
     return rc;
   GemmArgs p{};
@@ -883,18 +883,18 @@ int eimoe_experts(const void* x, int M, int H, int I, int H_out, const void* w_g
   int32_t* offsets = static_cast<int32_t*>(at(L.offsets));
   int32_t* rows = static_cast<int32_t*>(at(L.rows));
   int32_t* pos = static_cast<int32_t*>(at(L.pos));
-  // one source rank: the rows are grouped by expert already
+  // One source rank: the rows are grouped by expert already.  Rows of x past the counted ones get zeros in y
+  // (from the combine where there are planes).
   const bool merged = n_seg > n_local;
-  if (merged || L.planes) {
-    if ((rc = hip_check(launch_merge_segments(counts, n_seg, n_local, M, offsets, rows, pos, s), "merge segments")))
-      return rc;
-  } else if ((rc = hip_check(launch_counts_to_offsets(counts, n_seg, offsets, s), "counts_to_offsets"))) {
+  const bool maps = merged || L.planes;
+  const int y_dtype = w_dtype == EIMOE_F32 ? EIMOE_F32 : EIMOE_BF16;
+  if ((rc = hip_check(launch_merge_segments(counts, n_seg, n_local, M, offsets, maps ? rows : nullptr,
+                                            maps ? pos : nullptr, L.planes ? nullptr : y, H_out * elem_size(y_dtype), s),
+                      "merge segments")))
     return rc;
-  }
   if ((rc = run_gate_up(x, merged ? rows : nullptr, M, H, w_gate_up, w_dtype, w_gate_up_scale, H, I, offsets, n_local,
                         n_local, M, at(L.h), EIMOE_TILE_AUTO, s)))
     return rc;
-  const int y_dtype = w_dtype == EIMOE_F32 ? EIMOE_F32 : EIMOE_BF16;
   if (!L.planes)
     return run_down(at(L.h), I, w_down, w_dtype, w_down_scale, H_out, offsets, n_local, n_local, M, y, y_dtype, 1,
                     EIMOE_TILE_AUTO, s, nullptr, 0, merged ? rows : nullptr);

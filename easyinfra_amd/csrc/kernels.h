@@ -90,9 +90,10 @@ hipError_t launch_route_align(const float* logits, int T, int E, int k, int reno
                               int32_t* sorted_tok, int32_t* pos, int32_t* hist, hipStream_t s);
 hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offsets, hipStream_t s);
 // Segments (source rank, expert) regrouped by expert: merged bounds, merged -> original row and back
-// (S <= kMaxSeg, a multiple of n_exp; rows and pos hold max_rows entries).
+// (S <= kMaxSeg, a multiple of n_exp; rows and pos hold max_rows entries, or are both null where S = n_exp).  tail (may be
+// null): max_rows rows of tail_bytes (a multiple of 4), zeroed past the last segment.
 hipError_t launch_merge_segments(const int32_t* counts, int S, int n_exp, int max_rows, int32_t* offsets,
-                                 int32_t* rows, int32_t* pos, hipStream_t s);
+                                 int32_t* rows, int32_t* pos, void* tail, int tail_bytes, hipStream_t s);
 // MoE prologue: residual add + RMSNorm (+ router logits).  Routers of at most
 // kPrologueFusedMaxE experts and kPrologueFusedMaxGate bytes of gate weights are dotted in
 // the same pass; others (E % 64 == 0) go through the grouped GEMM with the T rows as one

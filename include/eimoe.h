@@ -191,8 +191,9 @@ int eimoe_gemm_down_w8a8(const void* hq, const float* h_scale, int I, const void
 /* The experts' MLP on pre-grouped rows: FusedMoE.forward_ep(hidden_states, expert_count)
  * (fused_moe.py:106-156), unweighted.  x [M, H] holds the rows of segment s = rank * n_local + e one
  * after the other, counts[s] each (device int32, n_seg a multiple of n_local); y [M, H_out] keeps
- * their order.  A negative count is an empty segment, and rows past M are left out.  Rows of one
- * expert from several source ranks are computed as one segment, so its
+ * their order.  A negative count is an empty segment; where the counts come to fewer than M rows the
+ * rest of y is zeros, and rows past M are left out.  Rows of one expert from several source ranks are
+ * computed as one segment, so its
  * weights are read once.  w_gate_up [n_local, 2I, H], w_down [n_local, H_out, I]: bf16 or fp8 (with
  * channel scales) and x, y bf16; or all fp32.  h is rounded to bf16 (fp32 experts: fp32), y once from
  * the fp32 sums.  H, I, H_out multiples of 64.  workspace: eimoe_experts_workspace_bytes bytes. */
@@ -222,7 +223,7 @@ int eimoe_grouped_gemm_ptrs(const void* a, const int32_t* a_rows, int a_nrows, i
 /* The op point's grouped GEMM where its list repeats the same n_b weights once per source rank: block
  * s of A holds counts[s] rows (device int32, n_seg a multiple of n_b) and multiplies b_ptrs[s % n_b];
  * c [M, N] bf16 keeps A's row order.  Blocks of one weight are computed as one segment, so a weight is
- * read once however many ranks sent rows.  Same operands and limits as eimoe_grouped_gemm_ptrs;
+ * read once however many ranks sent rows.  Rows of c past the counted ones are not written.  Same operands and limits as eimoe_grouped_gemm_ptrs;
  * workspace: eimoe_grouped_gemm_blocks_workspace_bytes bytes. */
 size_t eimoe_grouped_gemm_blocks_workspace_bytes(int M, int n_b);
 int eimoe_grouped_gemm_blocks(const void* a, int M, int lda, const void* const* b_ptrs, int n_b, int N, int K,

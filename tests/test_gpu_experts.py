@@ -138,17 +138,18 @@ def test_experts_tile_bounds(dev, E, H, I, rows, mode):
     assert oracle.rel_l2(y.cpu().float(), ref.cpu()) <= 2.0 ** -8
 
 
-# Counts that come to more rows than x has, or that are negative (empty segments), on each route that
-# regroups the rows: straight to their places, fp32 planes, K split planes.
+# Counts that come to fewer rows than x has, to more, or that are negative (empty segments), on each route:
+# rows straight to their places from one rank and from several, fp32 planes, K split planes.  Every row of
+# y is defined: its segment's product, or zeros past the last segment.
 @pytest.mark.gpu
-@pytest.mark.parametrize("E,ep,H,I", [(4, 2, 128, 128), (2, 2, 1024, 16384), (1, 1, 1024, 16384)])
-@pytest.mark.parametrize("kind", ["over", "negative"])
+@pytest.mark.parametrize("E,ep,H,I", [(4, 1, 128, 128), (4, 2, 128, 128), (2, 2, 1024, 16384), (1, 1, 1024, 16384)])
+@pytest.mark.parametrize("kind", ["short", "empty", "over", "negative"])
 @pytest.mark.parametrize("mode", ["bf16", "fp32"])
 def test_experts_counts_off_the_rows(dev, E, ep, H, I, kind, mode):
     M = 120
     g = torch.Generator().manual_seed(E * ep)
     S = E * ep
-    counts = torch.full((S,), {"over": 150 // S, "negative": 60 // S}[kind])
+    counts = torch.full((S,), {"short": 90 // S, "empty": 0, "over": 150 // S, "negative": 60 // S}[kind])
     if kind == "over":
         counts[0] = 2 ** 31 - 1 if S == 1 else counts[0]
         counts[-1] = 2 ** 31 - 1
@@ -167,5 +168,7 @@ def test_experts_counts_off_the_rows(dev, E, ep, H, I, kind, mode):
         ref[r:r + n] = oracle.expert_mlp(x[r:r + n].float(), wgu[s % E].float(), wd[s % E].float(),
                                          round_h_bf16=mode != "fp32")
         r += n
+    got = y.cpu().float()
+    assert not got[r:].any()
     # the bounds of test_experts_match_oracle_per_segment
-    assert float((y.cpu().float() - ref)[:r].norm()) <= (2e-5 if mode == "fp32" else 2.0 ** -8) * float(ref.norm())
+    assert float((got - ref).norm()) <= (2e-5 if mode == "fp32" else 2.0 ** -8) * float(ref.norm())
