@@ -2449,9 +2449,13 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
     else if (silu) t = avg < 0.7 ? kTileXS : avg < 25 ? kTileS : avg < 64 ? kTileMS : kTileL;
     // a launch as wide as a gate/up (four rounds of column tiles; no K split): the op point, 8 Mixtral-8x7B
     // weights (28672 x 4096), one hot, cold, 8 / 31 / 64 / 128 / 256 / 512 rows 166 / 297 / 330 / 342 / 381 / 406 us
-    // on 128x128, 157 / 266 / 289 / 307 / 318 / 389 on 64x128, 171 / 308 / 324 / 329 / 308 / 333 on 256x256
+    // on 128x128, 157 / 266 / 289 / 307 / 318 / 389 on 64x128, 171 / 308 / 324 / 329 / 308 / 333 on 256x256.
+    // 256x256 puts the hot weight's tall tiles on one XCD and loses to both until its rows (half of all) fill
+    // a second one: the call at 320 / 360 / 400 / 430 rows 383 / 381 / 377 / 377 on 128x128, 343 / 349 / 377 / 376
+    // on 64x128, 384 / 386 / 405 / 394 on 256x256, at 460 rows 375 / 407 / 393, at 520 rows 424 / - / 373; even
+    // rows, the GEMM at 300 / 420 / 512 rows 331 / 343 / 360, 310 / 320 / 386, 331 / 340 / 343
     else if (S >= 8 && p.k_split == 1 && static_cast<long long>(S) * (p.N / 128) >= 4 * kNumCu)
-      t = avg < 0.7 ? kTileXS : avg < 24 ? kTileMS : kTileL;
+      t = avg < 0.7 ? kTileXS : avg < 56 ? kTileMS : avg < 62 ? kTileM : kTileL;
     else t = avg < 0.7 ? kTileXS : avg < 128 ? kTileM : kTileL;
   } else if (silu) {
     // From the row bound, not the expected rows: the Qwen3-30B-A3B 32-expert share at 2048
