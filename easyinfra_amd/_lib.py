@@ -52,6 +52,7 @@ SIGNATURES = {
     "eimoe_experts_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "eimoe_experts": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p,
                               c_void_p, c_int, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "eimoe_gemm_tile": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "eimoe_grouped_gemm_blocks_workspace_bytes": (c_size_t, [c_int, c_int]),
     "eimoe_grouped_gemm_blocks": (c_int, [c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_int,
                                           c_void_p, c_void_p, c_size_t, c_void_p]),

@@ -720,6 +720,22 @@ int eimoe_grouped_gemm_blocks(const void* a, int M, int lda, const void* const* 
                            m.offsets, n_b, n_b, M, c, EIMOE_BF16, EIMOE_TILE_AUTO, stream, &m);
 }
 
+int eimoe_gemm_tile(int max_rows, int n_seg, int N, int K, int w_dtype, int gate_up, int k_split) {
+  if (max_rows < 1 || n_seg < 1 || n_seg > EIMOE_MAX_SEGMENTS || (w_dtype != EIMOE_BF16 && w_dtype != EIMOE_FP8))
+    return EIMOE_TILE_AUTO;
+  const int n_unit = gate_up ? 32 : 64;
+  if (N < n_unit || N % n_unit || k_split < 1 || k_split > 64 || K < 64 || K % (64 * k_split)) return EIMOE_TILE_AUTO;
+  GemmArgs p{};
+  p.max_rows = max_rows;
+  p.S = n_seg;
+  p.N = N;
+  p.nb_rows = gate_up ? 2 * N : N;
+  p.K = K / k_split;
+  p.k_split = k_split;
+  return gemm_choose_tile(p, gate_up ? kEpiSiluBF16 : k_split > 1 ? kEpiStoreF32 : kEpiStoreBF16, w_dtype == EIMOE_FP8,
+                          false);
+}
+
 int eimoe_combine(const void* y, int y_dtype, int n_split, long long split_stride, const int32_t* pos,
                   const float* topk_weights, int T, int k, int H, const void* shared_y, int shared_dtype, void* out,
                   int out_dtype, void* stream) {

@@ -278,6 +278,12 @@ size_t eimoe_fused_moe_workspace_bytes(int T, int H, int I, int E, int k, int n_
 int eimoe_fused_moe_down_split(int T, int H, int I, int E, int k, int n_local, int shared_inter, int out_dtype,
                                int flags);
 
+/* The tile (EIMOE_TILE_*) that automatic selection takes for a grouped GEMM of bf16 rows with bf16 or fp8
+ * weights: max_rows rows in n_seg segments, N output columns (gate_up: of each of the two halves), K in all,
+ * k_split slices of it.  No counterpart in the reference; for callers and tests that must know which kernel a
+ * size runs on.  Returns EIMOE_TILE_AUTO for arguments that the GEMM entry points refuse. */
+int eimoe_gemm_tile(int max_rows, int n_seg, int N, int K, int w_dtype, int gate_up, int k_split);
+
 /* The whole layer: hidden_states, router logits and top_k in, combined output out.
  * Composes router -> align -> gate/up+SiLU (gathering x rows directly) -> down -> combine
  * (+ shared experts), i.e. MoeAll2AllBlock's stages at ep=1 (blocks/moe/moe_all2all.py:85-95)

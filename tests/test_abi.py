@@ -193,6 +193,21 @@ def test_fused_down_split_query():
     assert L.eimoe_fused_moe_down_split(16, 256, 128, 8, 0, 8, 0, _lib.BF16, 1) == 0
 
 
+def test_gemm_tile_query():
+    """eimoe_gemm_tile: a tile whose columns divide N for sizes the GEMMs take, EIMOE_TILE_AUTO otherwise."""
+    f = _lib.lib().eimoe_gemm_tile
+    cols = {1: 256, 2: 128, 3: 128, 4: 64, 5: 32, 6: 128}
+    for n_seg, N, K in [(8, 14336, 4096), (64, 1408, 2048), (32, 2048, 768), (1, 4096, 14336), (2, 192, 64)]:
+        for dt in (_lib.BF16, _lib.FP8):
+            for gate_up in (0, 1):
+                for rows in (1, 7, 64, 500, 9000):
+                    t = f(rows, n_seg, N, K, dt, gate_up, 1)
+                    assert t in cols and N % (cols[t] // (2 if gate_up else 1)) == 0
+    assert f(0, 8, 128, 128, _lib.BF16, 0, 1) == 0 and f(8, 2000, 128, 128, _lib.BF16, 0, 1) == 0
+    assert f(8, 8, 100, 128, _lib.BF16, 0, 1) == 0 and f(8, 8, 128, 96, _lib.BF16, 0, 1) == 0
+    assert f(8, 8, 128, 128, _lib.F32, 0, 1) == 0 and f(8, 8, 128, 128, _lib.BF16, 0, 4) == 0
+
+
 def test_static_scratch_limit_matches_the_documented_token_count():
     """The largest Mixtral-8x7B layer (H 4096, I 14336, 8 experts, top-2) the 64 MiB static scratch
     holds, as the header states it: 545 tokens with bf16 or fp32 output."""

@@ -172,3 +172,77 @@ def test_experts_counts_off_the_rows(dev, E, ep, H, I, kind, mode):
     assert not got[r:].any()
     # the bounds of test_experts_match_oracle_per_segment
     assert float((got - ref).norm()) <= (2e-5 if mode == "fp32" else 2.0 ** -8) * float(ref.norm())
+
+
+L, M, S, XS, STREAM, MS = 1, 2, 3, 4, 5, 6   # EIMOE_TILE_*
+
+
+def _mapped_rows(E, ep, rows, seed):
+    """Rows of (source rank, expert), uneven, so that tiles end in remainders on every expert."""
+    g = torch.Generator().manual_seed(seed)
+    return torch.bincount(torch.randint(0, E * ep, (rows,), generator=g), minlength=E * ep)
+
+
+# Every kernel that stores rows through the map of merged ranks, with remainder tiles: the down projection on
+# each tile (in one round and past it, where ring and two-stage kernels meet; up to 64 experts and beyond,
+# where the 256x256 kernels change; W8A16 with K a multiple of 128 and not).  The tile is asserted, so that a
+# change of the rules moves the sizes here too.
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,H,I,per,mode,tile", [
+    (16, 2048, 256, 0.5, "bf16", STREAM), (16, 2048, 256, 5, "bf16", XS), (4, 512, 256, 40, "bf16", S),
+    (16, 2048, 256, 30, "bf16", MS), (32, 2048, 256, 35, "bf16", MS), (16, 1024, 256, 90, "bf16", M),
+    (16, 2048, 256, 45, "bf16", L), (16, 2048, 256, 300, "bf16", L), (70, 1024, 256, 210, "bf16", L),
+    (16, 2048, 256, 0.5, "w8a16", STREAM), (16, 2048, 256, 1.5, "w8a16", XS), (16, 2048, 256, 15, "w8a16", S),
+    (16, 2048, 256, 45, "w8a16", MS), (32, 2048, 256, 60, "w8a16", MS), (16, 2048, 256, 120, "w8a16", M),
+    (16, 2048, 256, 270, "w8a16", L), (70, 1024, 256, 400, "w8a16", L), (16, 2048, 192, 15, "w8a16", S),
+    (16, 2048, 192, 120, "w8a16", M)])
+def test_experts_store_through_the_map(dev, E, H, I, per, mode, tile):
+    ep, rows = 2, int(per * E)
+    dt = _lib.FP8 if mode == "w8a16" else _lib.BF16
+    assert _lib.lib().eimoe_gemm_tile(rows, E, H, I, dt, 0, 1) == tile
+    g = torch.Generator().manual_seed(E + rows)
+    counts = _mapped_rows(E, ep, rows, E + rows)
+    x = torch.randn(rows, H, generator=g).to(torch.bfloat16)
+    wgu = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(torch.bfloat16)
+    wd = (torch.randn(E, H, I, generator=g) * 0.05).to(torch.bfloat16)
+    ref_gu, ref_d, scales = wgu.float(), wd.float(), None
+    if mode == "w8a16":
+        (wgu, sgu), (wd, sd) = oracle.quantize_weights_fp8(wgu.float()), oracle.quantize_weights_fp8(wd.float())
+        ref_gu, ref_d = wgu.float() * sgu[..., None], wd.float() * sd[..., None]
+        scales = (sgu.to(dev), sd.to(dev))
+    print("CASE", dict(E=E, H=H, I=I, rows=rows, mode=mode, tile=tile), flush=True)
+    y = ops.experts(x.to(dev), wgu.to(dev), wd.to(dev), counts.to(torch.int32).to(dev), E, scales)
+    xd, rgu, rd = x.to(dev).float(), ref_gu.to(dev), ref_d.to(dev)
+    ref, r = torch.empty(rows, H, device=dev), 0
+    for s, c in enumerate(counts.tolist()):
+        gu = xd[r:r + c] @ rgu[s % E].T
+        h = (torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]).to(torch.bfloat16).float()
+        ref[r:r + c] = h @ rd[s % E].T
+        r += c
+    # as test_experts_tile_bounds, and row by row: a row in another's place is off by its whole size (a bf16
+    # rounding of one value is at most 2^-8 of it; h flips and the rest are far below)
+    err = (y.float() - ref).norm(dim=1)
+    assert bool((err <= 2.0 ** -7 * ref.norm(dim=1)).all())
+    assert oracle.rel_l2(y.cpu().float(), ref.cpu()) <= 2.0 ** -8
+
+
+# The op point on weights of 32 MiB over two ranks, both sides of each of its rule's bounds (56 and 62 rows per
+# weight), which are also the tiles that store through the map there.
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,tile", [(240, MS), (447, MS), (448, M), (495, M), (496, L), (1500, L)])
+def test_op_point_large_weights_store_through_the_map(dev, rows, tile):
+    import easyinfra_amd.torch_ops  # noqa: F401
+    E, ep, N, K = 8, 2, 16384, 1024
+    assert _lib.lib().eimoe_gemm_tile(rows, E, N, K, _lib.BF16, 0, 1) == tile
+    g = torch.Generator().manual_seed(rows)
+    blocks = _mapped_rows(E, ep, rows, rows).tolist()
+    a = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(dev)
+    w = [(torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16).to(dev) for _ in range(E)]
+    print("CASE", dict(rows=rows, tile=tile), flush=True)
+    out = torch.ops.ops.hip_grouped_gemm_single(a, w * ep, blocks)
+    r = 0
+    for s, c in enumerate(blocks):
+        ref = a[r:r + c].float() @ w[s % E].float().T
+        # one bf16 rounding, at most 2^-9 of each value; fp32 sums of 1024 terms
+        assert bool(((out[r:r + c].float() - ref).norm(dim=1) <= 2.0 ** -8 * ref.norm(dim=1)).all())
+        r += c
