@@ -1022,12 +1022,17 @@ int fused_moe_impl(const void* x, const float* logits, int T, int H, int I, int 
                             static_cast<long long>(H) * I * 2 <= 4ll * 1024 * 1024;
   // Shared experts (every token, weight 1) depend only on x: forked onto the second stream, to run beside
   // the routed GEMMs; joined before the combine.  The routing is launched first, and the fork waits for
-  // it, unless the shared gate/up leaves CUs to the small routing kernels (128x128 tiles at most the CUs):
-  // then it runs while the routing leaves the GPU idle (DeepSeek-V2-Lite, fork after -> before the
-  // routing, cold, one box: 150 tokens 178 -> 166 us; with the GPU filled 1200 tokens 335 -> 339).  W8A8
-  // layers, whose routed path also quantises x first, fork before it at any size (100 / 1000 tokens
-  // 150 -> 123 / 236 -> 225 us).
-  const bool fork_early = (flags & EIMOE_W8A8) || static_cast<long long>((T + 127) / 128) * (shared_inter / 64) <= kNumCu;
+  // it, unless the routed gate/up makes two rounds of the CUs (its 256x256 tiles at one m-tile per expert): then
+  // the shared experts run while the routing leaves the GPU idle, on W8A8 layers, whose routed path also quantises
+  // x first, at any size, on others while their gate/up leaves CUs to the small routing kernels (128x128 tiles at
+  // most the CUs).  DeepSeek-V2-Lite (2.75 rounds), fork after -> before the routing, one box: 150 / 220 / 330 tokens
+  // 181 -> 174 / 192 -> 189 / 227 -> 218 us, with the GPU filled 1200 tokens 335 -> 339; W8A8 100 / 500 / 1500 / 3500 tokens
+  // 142 -> 131 / 187 -> 176 / 269 -> 257 / 437 -> 420.  Where the routed launch makes one round, what the shared experts
+  // hold of it becomes a second: 32 experts of 3072 x 1024 and one shared at 300 / 1313 / 1700 tokens 161 -> 168 / 238 ->
+  // 275 / 268 -> 300, W8A8 at 1400 tokens 194 -> 219.
+  const bool two_rounds = static_cast<long long>(n_local) * (I / 128) >= 2 * kNumCu;
+  const bool fork_early = two_rounds && ((flags & EIMOE_W8A8) ||
+                                         static_cast<long long>((T + 127) / 128) * (shared_inter / 64) <= kNumCu);
   const void* sh_y = nullptr;
   AuxStream* aux = nullptr;
   if (shared_inter > 0 && !no_alloc) {

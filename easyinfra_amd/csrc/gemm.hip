@@ -833,7 +833,8 @@ grouped_gemm_dma_kernel(GemmArgs p) {
     if constexpr (F32 && BM >= kSplit3MinRows) {
       // Operands that do not fit their three terms lose bits; infinite and NaN operands (and products past
       // the fp32 range) leave sums that are not finite, as on the fp32 MFMA but not the same ones (inf * 0
-      // among the split terms).  Such a tile is computed again on the fp32 MFMA.  The vote is also the barrier before the stages are reused.
+      // among the split terms).  Such a tile is computed again on the fp32 MFMA.  The vote is also the barrier
+      // before the stages are reused.
       k_loop.template operator()<kSlabSplit3>();
       if (__syncthreads_or(split3_doubtful<G, MBE>(acc, lost) ? 1 : 0)) k_loop.template operator()<kSlabF32>();
     } else {
@@ -2324,58 +2325,47 @@ int gemm_out_cols_per_tile(int tile, int epi) {
   return epi_silu(epi) ? bn / 2 : bn;
 }
 
-// Routed launches (8 or more segments) of bf16 experts that stay in cache, from 8 to a few
-// hundred expected rows per segment.  What decides is whether a tile shape spreads the weight
-// panels over all CUs: the 256x256 tile is the fastest per tile (persistent, ping-pong) but with
-// few experts and narrow outputs it leaves CUs idle, the 64x128 tile (three workgroups per CU,
-// one m-tile for most segments) covers the CUs where 128x128 makes too few tiles and 32x128 reads
-// each weight panel once per 32 rows.  Tile counts are estimated at the expected rows.  Measured
-// per GEMM, single launches on the routed segments (cold, one box; us):
-//  * Qwen3-30B-A3B 32-expert share, 768 tokens (46 rows per expert, 198 at most): gate/up 52.8 on
-//    64x128 against 63.2 / 63.7 / 62.7 on 128x128 / 32x128 / 256x256, down 35.9 against 49.1 /
-//    48.2 / 41.4; 256 tokens (15 rows): gate/up 51.0 on 32x128 (64x128 52.9, 128x128 54.4), down
-//    33.4 on 128x128 (32x128 34.9);
-//  * DeepSeek-V2-Lite, 768 tokens (72 rows, zipf routing): gate/up 152.9 on 256x256 against
-//    174.3 / 178.6 / 218.9 on 64x128 / 128x128 / 32x128, down 88.2 against 99.5 / 105.1 / 115.3
-//    (uniform routing: 168.7 and 87.2 on 256x256); 128 tokens (12 rows): gate/up 112.6 on 128x128
-//    against 125.3 streamed and 128.4 on 32x128.
-// bf16 since the 64x128 tile runs on the ring, on segments an eighth of which hold 8 times the rows of the
-// others (cold, one box; us; expected rows per segment in brackets): gate/up, Qwen3 share 512 / 2048 / 4100
-// rows [16 / 64 / 128] 40.9 / 55.6 / 61.7 on 64x128, 48.8 / 52.2 / 75.7 on 128x128, 46.4 / 44.6 / 46.3 on
-// 256x256 (one round of 240 tiles); 16 DeepSeek-V2-Lite experts 256 / 1024 / 2048 rows [16 / 64 / 128] 37.5 /
-// 54.9 / 70.5, 45.9 / 50.2 / 73.0 and 43.9 / 41.7 / 44.1.  A 256x256 tile takes about the same time whatever
-// its height, so it wins once the rows would need a second round of the small tiles, down to half a
-// round of tiles.
+// Launches of 8 or more segments of experts that stay in cache, bf16 or W8A8: what decides is how many rounds
+// of the CUs a tile shape makes.  A 256x256 tile (persistent, ping-pong) takes about the same time whatever
+// its height, so it wins once the rows would need a second round of the small tiles; the 64x128 tile (on the
+// ring, one m-tile for most segments) covers the CUs below, where 32x128 (t) reads each weight panel once per
+// 32 rows.  Tile counts are estimated at the expected rows.
+// The bounds come from a sweep of 12 shapes (8-128 experts of 2048-4096 x 768-2048) at 6-330 expected rows, routed
+// evenly, zipf and with an eighth of the segments 8 times as popular (single GEMMs, cold, one box; us, the mean of the
+// three; rows in brackets): over all of it the gate/up is within 3.3 % (W8A8 3.5 %) of each size's best tile.
+// Gate/up to 256 rows of the bound: 256x256 where its tiles fill the CUs from 40 rows (64 DeepSeek-V2-Lite experts), in
+// half a round and more from 56: 16 experts of 2048 x 1024 [43] 38.6 against 33.4 on 64x128, W8A8 24.7 against 19.0, the
+// Qwen3 share [43] 42.4 against 40.9 and 26.0 against 22.3; one eighth hot [64 / 128] 44.6 / 46.3 against 55.6 / 61.7.
 static int routed_small_gate_up_tile(const GemmArgs& p, int S, double avg, int t) {
   const long long tiles_l = static_cast<long long>(S) * static_cast<long long>((avg + 255) / 256) * (p.N / 128);
   const long long tiles_m = static_cast<long long>(S) * static_cast<long long>((avg + 127) / 128) * (p.N / 64);
-  if (avg >= 40 && tiles_l >= kNumCu / 2) return kTileL;
+  if (avg >= (tiles_l >= kNumCu ? 40 : 56) && tiles_l >= kNumCu / 2) return kTileL;
   return avg >= (tiles_m >= 2 * kNumCu ? 8 : 16) && avg < 64 ? kTileMS : t;
 }
 
-// e4m3 (W8A8) tiles do half the MFMA work per weight byte: the 64x128 band reaches to 80 rows, the
-// 256x256 tile takes over from 64, and below 40 rows the 32x128 tile (t) stays.
-// bf16 (as above, us on 64x128 / 128x128 / 256x256): down, Qwen3 share 1024 / 2048 / 8192 rows [32 / 64 / 256]
-// 24.2 / 35.8 / 23.9, 28.3 / 34.5 / 36.0 and 51.5 / 56.6 / 45.6; 32 DeepSeek-V2-Lite experts 2048 / 8192 rows
-// [64 / 256] 43.6 / 55.0 / 54.7 and 97.4 / 85.3 / 69.4; the op point (N 1536, K 2048) 512 / 2048 / 4100 rows
-// [16 / 64 / 128] 36.4 / 43.3 / 41.0, 56.1 / 45.7 / 41.6 and 66.3 / 76.0 / 44.9, over 64 weights (N 2816) 2048
-// rows [32] 137.7 / 182.0 / 134.9.  256x256 where its tiles, a quarter more than segments for the skew, make
-// one round or from two rounds on; between them its second round is nearly empty.
-static int routed_small_down_tile(const GemmArgs& p, int S, double avg, int t, bool fp8) {
+// The down projection, bf16 from 8 and W8A8 from 20 expected rows per segment to 384 (the same sweep; within 4.1 %,
+// W8A8 5 %, of the best tile).  bf16: 64x128 from 12 rows to 60 and 128x128 beyond, 256x256 from 40 rows with two rounds
+// of its tiles, from 56 where they make 0.6-0.8 of one (between the two its second round is nearly empty, below
+// it leaves CUs idle: 16 experts of 2048 x 1024, half a round, [43 / 90 / 170] 23.0 / 25.3 / 27.8 against 18.3 on 64x128,
+// 23.1 / 25.6 on 128x128) and from 200 with half a round.  64x128 to 72 rows lost 4 % on 48 experts of 2048 x 1536 [64].
+// W8A8 does half the MFMA work per weight byte: 64x128 to 60 rows, or to 80 in one round, 128x128 beyond, 256x256 from
+// 64 rows with three rounds of tiles (96 experts of 2560 x 1280 [128] 107 against 110), 130 with two, 200 with half a one.
+static int routed_small_down_tile(const GemmArgs& p, int S, double avg, bool fp8) {
   const long long tiles_ms = static_cast<long long>(S) * static_cast<long long>((avg + 63) / 64) * (p.N / 128);
   const long long tiles_l = static_cast<long long>(S) * static_cast<long long>((avg + 255) / 256) * (p.N / 256);
   if (!fp8) {
     // (below 12 rows the two are level, 18.4 each at 4 rows and 21.2 at 8, unless 128x128 makes no more tiles than
     // CUs: 16 experts, 128 rows 23.9 -> 17.9 us; the Qwen3 share's layer at 128 tokens is 2 us slower on 64x128)
     if (avg < 40) return avg >= 12 || static_cast<long long>(S) * (p.N / 128) <= kNumCu ? kTileMS : kTileM;
-    if (tiles_l >= kNumCu / 2 && (tiles_l * 5 <= kNumCu * 4 || tiles_l >= 2 * kNumCu || avg >= 200)) return kTileL;
-    return avg < 72 ? kTileMS : kTileM;
+    if (tiles_l >= 2 * kNumCu || (avg >= 200 && tiles_l >= kNumCu / 2) ||
+        (avg >= 56 && tiles_l * 10 >= kNumCu * 6 && tiles_l * 5 <= kNumCu * 4))
+      return kTileL;
+    return avg < 60 ? kTileMS : kTileM;
   }
-  // W8A8: 64 DeepSeek-V2-Lite experts 1500 / 3000 / 6000 / 9000 rows [23 / 47 / 94 / 141] 45.2 / 51.9 / 67.1 / 82.4, 46.0 /
-  // 55.4 / 55.3 / 63.7 and 46.1 / 49.4 / 65.2 / 64.5, Qwen3 share 8192 rows [256] 38.5, 40.7 and 32.2
-  if (tiles_l >= kNumCu / 2 && (avg >= 200 || (avg >= 130 && tiles_l >= 2 * kNumCu))) return kTileL;
-  if (avg >= 20 && avg < (tiles_ms <= 3 * kNumCu ? 80 : 60)) return kTileMS;   // 80: one round of 64x128 workgroups
-  return avg < 20 ? t : kTileM;
+  if ((tiles_l >= kNumCu / 2 && avg >= 200) || (tiles_l >= 2 * kNumCu && avg >= 130) ||
+      (tiles_l >= 3 * kNumCu && avg >= 64))
+    return kTileL;
+  return avg < (tiles_ms <= 3 * kNumCu ? 80 : 60) ? kTileMS : kTileM;   // 80: one round of 64x128 workgroups
 }
 
 // Down projections of one or two experts of >= 32 MiB (an expert-parallel share): their column tiles
@@ -2390,6 +2380,7 @@ static int routed_small_down_tile(const GemmArgs& p, int S, double avg, int t, b
 bool few_large_down(int S, int N, double expert_bytes) {
   return expert_bytes >= 32.0 * 1024 * 1024 && static_cast<long long>(S) * (N / 128) * 4 <= kNumCu;
 }
+// (Under 0.7 rows: one row over two experts or more.)
 int few_large_down_tile(int S, double avg) {
   return avg < 0.7 ? kTileXS : avg <= (S == 1 ? 36 : 24) ? kTileS : avg <= 192 ? kTileMS : kTileL;
 }
@@ -2405,8 +2396,8 @@ int few_large_down_tile(int S, double avg) {
 //    256x256 tile from ~256 rows per segment of the bound (DeepSeek 4096 tokens 717 vs 710
 //    us skewed, 580 vs 657 uniform against 128x128); the down projection (short K) wants
 //    more, smaller tiles: 128x128 below ~384 expected rows per segment (Qwen3 2048 tokens:
-//    46 vs 62 us), 32x128 below ~96.  Routed bf16 launches of 8 or more segments between 8
-//    and 384 expected rows take routed_small_gate_up_tile / routed_small_down_tile instead.
+//    46 vs 62 us), 32x128 below ~96.  Launches of 8 or more segments take
+//    routed_small_gate_up_tile / routed_small_down_tile in their ranges instead.
 int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
   const int S = p.S > 0 ? p.S : 1;
   const double avg_bound = static_cast<double>(p.max_rows) / S;
@@ -2422,7 +2413,7 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
   } else if (!b_fp8 && silu && known && S == 1 && expert_bytes >= 32.0 * 1024 * 1024) {
     // one expert: the rows are known, so the tile that holds them (Mixtral-8x7B, us, cold: 64 rows 62.3
     // on 128x128, 51.5 on 64x128; 511 rows, four m-tiles of 128, 157 against 90 on 256x256)
-    t = avg < 0.7 ? kTileXS : avg <= 32 ? kTileS : avg <= 64 ? kTileMS : avg <= 128 ? kTileM : kTileL;
+    t = avg <= 32 ? kTileS : avg <= 64 ? kTileMS : avg <= 128 ? kTileM : kTileL;
     idle_ok = true;
   } else if (expert_bytes >= 32.0 * 1024 * 1024) {
     // (W8A8 gate/up at 16 rows per expert on the routed, gathered rows of a Mixtral-8x7B
@@ -2465,7 +2456,7 @@ int gemm_pick_tile(const GemmArgs& p, int epi, bool b_fp8) {
     if (S >= 8 && avg_bound < 256) t = routed_small_gate_up_tile(p, S, avg, t);
   } else {
     t = avg < 6 ? kTileXS : avg < 96 ? kTileS : avg < 384 ? kTileM : kTileL;
-    if (S >= 8 && avg >= (b_fp8 ? 20 : 8) && avg < 384) t = routed_small_down_tile(p, S, avg, t, b_fp8);
+    if (S >= 8 && avg >= (b_fp8 ? 20 : 8) && avg < 384) t = routed_small_down_tile(p, S, avg, b_fp8);
   }
   if (t == kTileL) {
     // fewer 256x256 tiles than CUs (a dense shared-expert launch, say) leaves CUs idle: step down
@@ -2501,12 +2492,9 @@ int gemm_choose_tile(const GemmArgs& p, int epi, bool b_fp8, bool a_fp8) {
     // 257.3 / 140.5 on 64x128); layers at 4 / 8 / 32 / 64 / 128 tokens 206 / 207 / 273 / 293 / 327 ->
     // 185 / 190 / 233 / 260 / 302 us against streaming below 12 rows.
     // Experts that stay in cache read half the bytes of their bf16 form, so the smaller tiles keep
-    // the CUs busy longer: 16x64 from one row (not streamed), 32x128 from 4, 64x128 from 20, the
-    // down projection on 128x128 from 100 and both on 256x256 from 256 (gate/up / down us,
-    // single GEMMs, cold: Qwen3-30B-A3B share 256 tokens 26.1 / 17.9 on 32x128 against 37.3 /
-    // 22.8 streamed, 768 tokens 29.7 / 27.3 on 64x128 against 39.8 / 36.2 on 128x128, 2048 tokens
-    // 48.9 on 64x128 / 39.0 on 128x128 against 53.8 / 52.6 on 256x256; DeepSeek-V2-Lite 768 tokens
-    // 108.8 / 66.9 on 64x128 against 125.9 / 78.9 on 128x128).
+    // the CUs busy longer: 16x64 from one row (not streamed; single GEMMs, cold, gate/up / down us: Qwen3-30B-A3B
+    // share 256 tokens 26.1 / 17.9 on 32x128 against 37.3 / 22.8 streamed), 32x128 from 4; above that by the rounds of
+    // the 256x256 tile (its sweep as at routed_small_gate_up_tile: within 4.6 % of the best tile, down 5.7 %).
     // One large expert, whose rows are known: the gate/up on the tile that holds them (Mixtral-8x7B, cold,
     // us: 31 rows 35.7 -> 29.8 on 32x128, 64 / 128 rows 44.2 / 53.7 -> 36.4 / 45.9 on 64x128).
     const bool known = p.rows_hint <= 0;
@@ -2514,26 +2502,32 @@ int gemm_choose_tile(const GemmArgs& p, int epi, bool b_fp8, bool a_fp8) {
     if (few_down) {
       tile = few_large_down_tile(p.S, avg);
     } else if (expert_bytes >= 32.0 * 1024 * 1024 && epi_silu(epi) && known && p.S == 1) {
-      tile = avg < 1 ? kTileXS : avg <= 32 ? kTileS : avg <= 128 ? kTileMS : avg <= 256 ? kTileM : kTileL;
+      tile = avg <= 32 ? kTileS : avg <= 128 ? kTileMS : avg <= 256 ? kTileM : kTileL;
     } else if (expert_bytes >= 32.0 * 1024 * 1024) {
       tile = avg < 1 ? kTileXS : avg < 24 ? kTileS : avg < 56 ? kTileMS : avg < 128 ? kTileM : kTileL;
     } else {
-      // (segments an eighth of which hold 8 times the rows of the others, rows per segment in brackets: gate/up,
-      // Qwen3 share 4100 / 8192 rows [128 / 256] 60.5 / 103.3 on 64x128, 60.2 / 79.8 on 128x128, 49.1 / 91.1 on
-      // 256x256, 16 DeepSeek-V2-Lite experts 2048 / 4100 rows 60.5 / 101.9, 60.0 / 66.8 and 49.6 / 90.8, 32 of them
-      // 4100 / 8192 rows 104.9 / 188.5, 87.9 / 129.1 and 89.4 / 138.0; down, 1024 rows [32] 21.6 -> 16.9 and 29.7 -> 23.8
-      // on 32x128 against 64x128)
-      const bool one_round = static_cast<long long>(p.S) * (p.N / 128) * 5 <= 4 * kNumCu;   // of 256x256 gate/up tiles
-      // (64 DeepSeek-V2-Lite experts, layers: 2400 tokens [225] 593 -> 476 us on 128x128, 3300 [309] 550 -> 568;
-      // gate/up 1500 / 3000 / 6000 rows [23 / 47 / 94] 83.2 / 105.7 / 169.5 on 32x128, 103.9 / 115.9 / 148.6 on 64x128, 103.0 /
-      // 123.9 / 126.5 on 128x128; down 4600 / 6000 rows [72 / 94] 81.1 / 93.3 on 64x128, 73.6 / 73.5 on 128x128)
-      const bool two_rounds = static_cast<long long>(p.S) * (p.N / 128) >= 2 * kNumCu;
-      const bool wide = static_cast<long long>(p.S) * (p.N / 128) >= 4 * kNumCu;
-      if (epi_silu(epi))
-        tile = avg < 4 ? kTileXS : avg < (two_rounds ? 56 : 20) ? kTileS : avg < (two_rounds ? 56 : 100) ? kTileMS
-               : avg < 200 && one_round ? kTileL : avg < (two_rounds ? 256 : 384) ? kTileM : kTileL;
-      else
-        tile = avg < 4 ? kTileXS : avg < 40 ? kTileS : avg < (wide ? 60 : 100) ? kTileMS : avg < 256 ? kTileM : kTileL;
+      // Gate/up: 64x128 to 100 rows, then 256x256 where it makes one round, filled to 0.6 or more, until the rows make
+      // a second m-tile (200), else 128x128 (64x128 while that leaves CUs idle: 8 experts of 3072 x 1536 [128] 38 against
+      // 49); 256x256 again from 256 rows where it still makes one round (16 of 2048 x 1024 [256 / 330] 49 / 50 against 57 /
+      // 64), from 300 (32 DeepSeek-V2-Lite experts [256 / 330] 136 / 139 against 122 / 148) or from 384 (the Qwen3 share
+      // [256 / 330] 91 / 92 against 76 / 89).  Launches of two rounds of 256x256 tiles: 32x128 to 56 rows (64 DeepSeek-V2-Lite
+      // experts, one eighth hot, [20 / 43] 86 / 105 against 103 / 115 on 64x128), then 128x128 to 256.
+      const long long tiles = static_cast<long long>(p.S) * (p.N / 128);   // 256x256 gate/up tiles, one m-tile each
+      const bool one_round = tiles * 5 <= 4 * kNumCu;
+      const bool two_rounds = tiles >= 2 * kNumCu;
+      if (epi_silu(epi)) {
+        if (avg < (two_rounds ? 56 : 20)) tile = avg < 4 ? kTileXS : kTileS;
+        else if (avg < (two_rounds ? 56 : 100)) tile = kTileMS;
+        else if (avg < 200 && one_round && tiles * 5 >= 3 * kNumCu) tile = kTileL;
+        else if (avg < 150 && static_cast<long long>(p.S) * (p.N / 64) < kNumCu) tile = kTileMS;
+        else tile = avg < (two_rounds || tiles * 2 <= kNumCu ? 256 : one_round ? 384 : 300) ? kTileM : kTileL;
+      } else {
+        // Down: 32x128 to 40 rows (the Qwen3 share, one eighth hot, [32] 18.2 against 23.6 on 64x128), to 20 where its column
+        // tiles make 1.5 rounds or fewer (12 experts of 4096 x 2048 [32] 33.4 against 25.1, 8 of 3072 x 1536 18.0 against
+        // 14.3), 64x128 to 100 (60 from four rounds on: 64 DeepSeek-V2-Lite experts), 128x128 to 256.
+        tile = avg < 4 ? kTileXS : avg < (tiles * 2 <= 3 * kNumCu ? 20 : 40) ? kTileS
+               : avg < (tiles >= 4 * kNumCu ? 60 : 100) ? kTileMS : avg < 256 ? kTileM : kTileL;
+      }
       keep_xs = avg >= 1;
     }
     if (tile == kTileL && !few_down &&

@@ -60,7 +60,7 @@ def test_layer_small_variant(dev, name, T):
     assert float((got - ref).abs().max()) <= 2e-2
     if inp.x.dtype == torch.bfloat16:
         assert float((got - tight).abs().max()) <= 2e-3 * max(1.0, float(tight.abs().max()))
-    else:   # the fp32 layer: fp32 operands on the fp32 MFMA, only the summation order differs
+    else:   # the fp32 layer: fp32's error, only the products' rounding and the summation order differ
         assert oracle.rel_l2(got, ref) <= 2e-5
         assert float((got - ref).abs().max()) <= 1e-4 * max(1.0, float(ref.abs().max()))
 
