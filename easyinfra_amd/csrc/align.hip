@@ -196,27 +196,46 @@ hipError_t launch_align(const int32_t* ids, int T, int k, int e_lo, int n_loc, i
 
 // Segments from a counts vector (the forward_ep entry: rows already grouped by
 // (src_rank, local_expert), fused_moe.py:395-439).  offsets = exclusive cumsum.
+// ROWS: of segments over max_rows rows, where a negative count is an empty segment and the bounds end at
+// max_rows (sums saturate there: with at most 2^24 rows, 2 GiB of 64 columns, nothing leaves 32 bits); the rows
+// past the last segment get tail_words words of zeros each in tail.
+template <bool ROWS>
 __global__ __launch_bounds__(64) void counts_to_offsets_kernel(const int32_t* __restrict__ counts, int S,
-                                                               int32_t* __restrict__ offsets) {
+                                                               int32_t* __restrict__ offsets, int max_rows,
+                                                               uint32_t* __restrict__ tail, int tail_words) {
   const int lane = threadIdx.x;
   const int per = (S + 63) / 64;
   const int b0 = lane * per;
+  auto count = [&](int s) { return ROWS ? min(max(counts[s], 0), max_rows) : counts[s]; };
+  auto bound = [&](int v) { return ROWS ? min(v, max_rows) : v; };
   int s = 0;
   for (int j = 0; j < per; ++j)
-    if (b0 + j < S) s += counts[b0 + j];
+    if (b0 + j < S) s = bound(s + count(b0 + j));
   const int incl = wave_incl_scan(s);
   int run = incl - s;
   for (int j = 0; j < per; ++j) {
     if (b0 + j < S) {
-      offsets[b0 + j] = run;
-      run += counts[b0 + j];
+      offsets[b0 + j] = bound(run);
+      run = bound(run) + count(b0 + j);
     }
   }
-  if (lane == 63) offsets[S] = incl;
+  const int end = bound(__shfl(incl, 63, 64));
+  if (lane == 63) offsets[S] = end;
+  if constexpr (ROWS)
+    for (int r = end; r < max_rows; ++r)
+      for (int i = lane; i < tail_words; i += 64) tail[static_cast<long long>(r) * tail_words + i] = 0u;
 }
 
 hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offsets, hipStream_t s) {
-  hipLaunchKernelGGL(counts_to_offsets_kernel, dim3(1), dim3(64), 0, s, counts, S, offsets);
+  hipLaunchKernelGGL(counts_to_offsets_kernel<false>, dim3(1), dim3(64), 0, s, counts, S, offsets, 0, nullptr, 0);
+  return hipGetLastError();
+}
+
+hipError_t launch_segment_bounds(const int32_t* counts, int S, int max_rows, int32_t* offsets, void* tail,
+                                 int tail_bytes, hipStream_t s) {
+  if (max_rows > (1 << 24)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(counts_to_offsets_kernel<true>, dim3(1), dim3(64), 0, s, counts, S, offsets, max_rows,
+                     static_cast<uint32_t*>(tail), tail_bytes / 4);
   return hipGetLastError();
 }
 
@@ -226,8 +245,7 @@ hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offse
 // expert is one segment.  offsets[n_exp + 1]: the experts' bounds in merged order; rows[m]: the
 // original row of merged row m; pos[r]: the merged row of original row r, -1 for rows past the last
 // segment, of which tail (null: left as it is) gets tail_words words of zeros each.  One launch (it stands
-// in for counts_to_offsets, ~4.5 us either way).  One source rank (S = n_exp) whose rows need no map: rows
-// and pos null, one workgroup.
+// in for counts_to_offsets, ~4.5 us either way).
 // A negative count stands for an empty segment and the bounds end at max_rows, so that segments never
 // overlap: every entry of pos is written, and every merged row below offsets[n_exp] names a row below
 // max_rows, whatever the counts say.
@@ -270,10 +288,6 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
   if (tail)
     for (int r = end + seg; r < max_rows; r += gridDim.x)
       for (int i = tid; i < tail_words; i += 256) tail[static_cast<long long>(r) * tail_words + i] = 0u;
-  if (!rows) {
-    for (int s = tid; s <= S; s += 256) offsets[s] = s_bound[s];
-    return;
-  }
   // of this thread's segments, the rows of those before `seg` in merged order (a lower expert, or the same
   // expert of a lower rank)
   const int e = seg % n_exp;
@@ -303,10 +317,9 @@ __global__ __launch_bounds__(256) void merge_segments_kernel(const int32_t* __re
 
 hipError_t launch_merge_segments(const int32_t* counts, int S, int n_exp, int max_rows, int32_t* offsets,
                                  int32_t* rows, int32_t* pos, void* tail, int tail_bytes, hipStream_t s) {
-  if (S < 1 || S > kMaxSeg || n_exp < 1 || S % n_exp != 0 || max_rows > (1 << 24) || !rows != !pos ||
-      (!rows && S != n_exp))
+  if (S < 1 || S > kMaxSeg || n_exp < 1 || S % n_exp != 0 || max_rows > (1 << 24))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(merge_segments_kernel, dim3(rows ? static_cast<unsigned>(S) : 1u), dim3(256), 0, s, counts, S, n_exp,
+  hipLaunchKernelGGL(merge_segments_kernel, dim3(static_cast<unsigned>(S)), dim3(256), 0, s, counts, S, n_exp,
                      max_rows, offsets, rows, pos, static_cast<uint32_t*>(tail), tail_bytes / 4);
   return hipGetLastError();
 }

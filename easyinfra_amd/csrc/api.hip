@@ -904,9 +904,11 @@ int eimoe_experts(const void* x, int M, int H, int I, int H_out, const void* w_g
   const bool merged = n_seg > n_local;
   const bool maps = merged || L.planes;
   const int y_dtype = w_dtype == EIMOE_F32 ? EIMOE_F32 : EIMOE_BF16;
-  if ((rc = hip_check(launch_merge_segments(counts, n_seg, n_local, M, offsets, maps ? rows : nullptr,
-                                            maps ? pos : nullptr, L.planes ? nullptr : y, H_out * elem_size(y_dtype), s),
-                      "merge segments")))
+  const int y_row = H_out * elem_size(y_dtype);
+  if ((rc = hip_check(maps ? launch_merge_segments(counts, n_seg, n_local, M, offsets, rows, pos,
+                                                   L.planes ? nullptr : y, y_row, s)
+                           : launch_segment_bounds(counts, n_seg, M, offsets, y, y_row, s),
+                      "segments")))
     return rc;
   if ((rc = run_gate_up(x, merged ? rows : nullptr, M, H, w_gate_up, w_dtype, w_gate_up_scale, H, I, offsets, n_local,
                         n_local, M, at(L.h), EIMOE_TILE_AUTO, s)))

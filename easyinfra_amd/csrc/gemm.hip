@@ -523,20 +523,15 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, const TileCoord& tc,
   const auto& cs = sc.cs;
   const auto& cs_up = sc.cs_up;
   const auto& rs = sc.rs;
-  // the output rows, all loaded before the first store (see EpiScales)
-  int out_row[EPI == kEpiStoreBF16 ? MBE : 1][4];
-  if constexpr (EPI == kEpiStoreBF16) {
+  // the mapped output rows, all loaded before the first store (see EpiScales)
+  constexpr bool MAPPED = EPI == kEpiStoreBF16Map;
+  int out_row[MAPPED ? MBE : 1][4];
+  if constexpr (MAPPED) {
 #pragma unroll
     for (int i = 0; i < MBE; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        out_row[i][r] = min(tc.row0 + wm * 16 * MBE + i * 16 + lq * 4 + r, tc.row_end - 1);
-    if (p.c_rows) {
-#pragma unroll
-      for (int i = 0; i < MBE; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) out_row[i][r] = p.c_rows[out_row[i][r]];
-    }
+        out_row[i][r] = p.c_rows[min(tc.row0 + wm * 16 * MBE + i * 16 + lq * 4 + r, tc.row_end - 1)];
   }
 #pragma unroll
   for (int i = 0; i < MBE; ++i) {
@@ -567,7 +562,7 @@ __device__ __forceinline__ void epilogue(const GemmArgs& p, const TileCoord& tc,
         float v[G::NI];
 #pragma unroll
         for (int j = 0; j < G::NI; ++j) v[j] = acc[i][j][r] * rs[i][r] * cs[j];
-        const int c_row = EPI == kEpiStoreBF16 ? out_row[EPI == kEpiStoreBF16 ? i : 0][r] : row;
+        const int c_row = MAPPED ? out_row[MAPPED ? i : 0][r] : row;
         const long long off =
             static_cast<long long>(tc.split) * p.c_split_stride + static_cast<long long>(c_row) * p.ldc + col0;
         if constexpr (EPI == kEpiStoreF32) {
@@ -2579,6 +2574,8 @@ hipError_t launch_grouped_gemm(const GemmArgs& p, int epi, bool b_fp8, bool a_fp
   }
   if (epi == kEpiSiluBF16) return b_fp8 ? launch_epi<kEpiSiluBF16, true>(q, max_rows, tile, a_fp8, s)
                                         : launch_epi<kEpiSiluBF16, false>(q, max_rows, tile, false, s);
+  if (epi == kEpiStoreBF16 && p.c_rows) return b_fp8 ? launch_epi<kEpiStoreBF16Map, true>(q, max_rows, tile, a_fp8, s)
+                                                     : launch_epi<kEpiStoreBF16Map, false>(q, max_rows, tile, false, s);
   if (epi == kEpiStoreBF16) return b_fp8 ? launch_epi<kEpiStoreBF16, true>(q, max_rows, tile, a_fp8, s)
                                          : launch_epi<kEpiStoreBF16, false>(q, max_rows, tile, false, s);
   return b_fp8 ? launch_epi<kEpiStoreF32, true>(q, max_rows, tile, a_fp8, s)

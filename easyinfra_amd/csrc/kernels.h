@@ -8,7 +8,9 @@ namespace eimoe {
 
 constexpr int kMaxSeg = 1024;  // segments (local experts x source ranks) per grouped GEMM
 
-enum Epilogue : int { kEpiStoreF32 = 0, kEpiStoreBF16 = 1, kEpiSiluBF16 = 2, kEpiSiluF32 = 3 };
+// kEpiStoreBF16Map: the bf16 store through GemmArgs::c_rows, in kernels of its own (its registers and loads in the
+// plain ones made a 48 us down projection on 64x128 tiles 5 % slower); picked by the launcher.
+enum Epilogue : int { kEpiStoreF32 = 0, kEpiStoreBF16 = 1, kEpiSiluBF16 = 2, kEpiSiluF32 = 3, kEpiStoreBF16Map = 4 };
 constexpr bool epi_silu(int epi) { return epi == kEpiSiluBF16 || epi == kEpiSiluF32; }
 
 // One grouped GEMM launch: for each segment s (rows [seg_off[s], seg_off[s+1]) of A),
@@ -89,8 +91,12 @@ hipError_t launch_route_align(const float* logits, int T, int E, int k, int reno
                               int32_t* ids, float* w, int32_t* counts, int32_t* offsets, int32_t* sorted_flat,
                               int32_t* sorted_tok, int32_t* pos, int32_t* hist, hipStream_t s);
 hipError_t launch_counts_to_offsets(const int32_t* counts, int S, int32_t* offsets, hipStream_t s);
+// The same for segments over max_rows rows: bounds that stay in range and never overlap whatever the counts, and
+// zeros in tail's rows (tail_bytes each, a multiple of 4) past the last segment.
+hipError_t launch_segment_bounds(const int32_t* counts, int S, int max_rows, int32_t* offsets, void* tail,
+                                 int tail_bytes, hipStream_t s);
 // Segments (source rank, expert) regrouped by expert: merged bounds, merged -> original row and back
-// (S <= kMaxSeg, a multiple of n_exp; rows and pos hold max_rows entries, or are both null where S = n_exp).  tail (may be
+// (S <= kMaxSeg, a multiple of n_exp; rows and pos hold max_rows entries).  tail (may be
 // null): max_rows rows of tail_bytes (a multiple of 4), zeroed past the last segment.
 hipError_t launch_merge_segments(const int32_t* counts, int S, int n_exp, int max_rows, int32_t* offsets,
                                  int32_t* rows, int32_t* pos, void* tail, int tail_bytes, hipStream_t s);

@@ -191,7 +191,7 @@ def _mapped_rows(E, ep, rows, seed):
 @pytest.mark.parametrize("E,H,I,per,mode,tile", [
     (16, 2048, 256, 0.5, "bf16", STREAM), (16, 2048, 256, 5, "bf16", XS), (4, 512, 256, 40, "bf16", S),
     (16, 2048, 256, 30, "bf16", MS), (32, 2048, 256, 35, "bf16", MS), (16, 1024, 256, 90, "bf16", M),
-    (16, 2048, 256, 45, "bf16", L), (16, 2048, 256, 300, "bf16", L), (70, 1024, 256, 210, "bf16", L),
+    (20, 2048, 256, 60, "bf16", L), (16, 2048, 256, 300, "bf16", L), (70, 1024, 256, 210, "bf16", L),
     (16, 2048, 256, 0.5, "w8a16", STREAM), (16, 2048, 256, 1.5, "w8a16", XS), (16, 2048, 256, 15, "w8a16", S),
     (16, 2048, 256, 45, "w8a16", MS), (32, 2048, 256, 60, "w8a16", MS), (16, 2048, 256, 120, "w8a16", M),
     (16, 2048, 256, 270, "w8a16", L), (70, 1024, 256, 400, "w8a16", L), (16, 2048, 192, 15, "w8a16", S),
