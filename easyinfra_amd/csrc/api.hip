@@ -180,6 +180,11 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
   if (tile == kTileL && work >= 4.0 * kNumCu) return 1;
   int best = 1;
   double best_cost = 1e300;
+  // A second plane has to pay.  On 256x256 tiles of routed small experts the rounds just past a whole one are an estimate (12
+  // experts of 4096 x 2048 at 250-330 rows each: 2 rounds or 1.5 and a plane, 8 % less by this count, 266.4 against 267.0 us
+  // measured for the layer at 1533 tokens), and the plane can take the layer past the static scratch.
+  const double bar =
+      tile == kTileL && n_local >= 8 && per < 384 && expert_bytes < 32.0 * 1024 * 1024 ? 0.9 : 0.98;
   for (int split = 1; split <= 8; split *= 2) {
     if (I % (64 * split) != 0) break;
     const long long items = tiles * split;
@@ -192,7 +197,7 @@ int pick_down_split(int max_rows, int rows_hint, int n_local, int H, int I, int 
     const double fill = one_seg ? 0.75 : n_local >= 8 && expert_bytes < 32.0 * 1024 * 1024 ? 0.4 : 1.0;
     const bool few = tile == kTileL ? work * split < fill * kNumCu : items < 2 * kNumCu;
     if (few && split < 8 && I % (128 * split) == 0) cost = 1e300;
-    if (cost < best_cost * 0.98) {
+    if (cost < best_cost * bar) {
       best_cost = cost;
       best = split;
     }
@@ -243,8 +248,9 @@ FusedLayout fused_layout(int T, int H, int I, int E, int k, int n_local, int Is,
   L.sorted_flat = take(A * 4);
   L.sorted_tok = take(A * 4);
   L.pos = take(A * 4);
-  L.hist = take(std::max(align_plan(static_cast<int>(A), n_local).hist_ints, route_hist_ints(T, E, k, n_local)) * 4);
-  L.h = take(A * I * hb);
+  // the routing's chunk counts lie in h, which the gate/up writes after the routing has read them
+  const size_t hist = std::max(align_plan(static_cast<int>(A), n_local).hist_ints, route_hist_ints(T, E, k, n_local)) * 4;
+  L.hist = L.h = take(std::max(A * I * hb, hist));
   if (L.h_terms == 2) L.h_lo = take(A * I * 2);
   L.y = take(static_cast<size_t>(L.h_terms) * L.k_split * A * H * elem_size(L.y_dtype));
   if (flags & EIMOE_W8A8) {

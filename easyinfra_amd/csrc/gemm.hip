@@ -2339,7 +2339,7 @@ static int routed_small_gate_up_tile(const GemmArgs& p, int S, double avg, int t
 }
 
 // The down projection, bf16 from 8 and W8A8 from 20 expected rows per segment to 384 (the same sweep; within 4.1 %,
-// W8A8 5 %, of the best tile).  bf16: 64x128 from 12 rows to 60 and 128x128 beyond, 256x256 from 40 rows with two rounds
+// W8A8 5 %, of the best tile).  bf16: 64x128 from 12 rows to 64 and 128x128 beyond, 256x256 from 40 rows with two rounds
 // of its tiles, from 56 where they make 0.6-0.8 of one (between the two its second round is nearly empty, below
 // it leaves CUs idle: 16 experts of 2048 x 1024, half a round, [43 / 90 / 170] 23.0 / 25.3 / 27.8 against 18.3 on 64x128,
 // 23.1 / 25.6 on 128x128) and from 200 with half a round.  64x128 to 72 rows lost 4 % on 48 experts of 2048 x 1536 [64].
@@ -2355,7 +2355,7 @@ static int routed_small_down_tile(const GemmArgs& p, int S, double avg, bool fp8
     if (tiles_l >= 2 * kNumCu || (avg >= 200 && tiles_l >= kNumCu / 2) ||
         (avg >= 56 && tiles_l * 10 >= kNumCu * 6 && tiles_l * 5 <= kNumCu * 4))
       return kTileL;
-    return avg < 60 ? kTileMS : kTileM;
+    return avg < 64 ? kTileMS : kTileM;
   }
   if ((tiles_l >= kNumCu / 2 && avg >= 200) || (tiles_l >= 2 * kNumCu && avg >= 130) ||
       (tiles_l >= 3 * kNumCu && avg >= 64))

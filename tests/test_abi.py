@@ -219,6 +219,17 @@ def test_static_scratch_limit_matches_the_documented_token_count():
         assert need(545) <= cap < need(546)
 
 
+@pytest.mark.parametrize("H,I,E,k,flags,lo,hi", [(4096, 2048, 12, 2, 1, 1499, 1632), (4096, 2816, 20, 2, 17, 600, 639),
+                                                 (1024, 1024, 16, 2, 5, 4354, 4354)])
+def test_static_scratch_holds_small_expert_layers(H, I, E, k, flags, lo, hi):
+    """Token counts at which a second K split plane, or the routing's chunk counts, would take a layer of small
+    experts past the static scratch (plain, H_SPLIT and W8A8)."""
+    L = _lib.lib()
+    for T in range(lo, hi + 1):
+        assert 0 < L.eimoe_fused_moe_workspace_bytes(T, H, I, E, k, E, 0, _lib.BF16, flags) <= \
+            L.eimoe_fused_moe_static_bytes()
+
+
 def test_ops_refuse_cpu_tensors():
     torch = pytest.importorskip("torch")
     from easyinfra_amd import ops
