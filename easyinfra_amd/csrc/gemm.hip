@@ -2334,7 +2334,11 @@ int gemm_out_cols_per_tile(int tile, int epi) {
 static int routed_small_gate_up_tile(const GemmArgs& p, int S, double avg, int t) {
   const long long tiles_l = static_cast<long long>(S) * static_cast<long long>((avg + 255) / 256) * (p.N / 128);
   const long long tiles_m = static_cast<long long>(S) * static_cast<long long>((avg + 127) / 128) * (p.N / 64);
-  if (avg >= (tiles_l >= kNumCu ? 40 : 56) && tiles_l >= kNumCu / 2) return kTileL;
+  // (just under 256 rows the segments past them take a second m-tile and the launch a second round: W8A8 layers of 12
+  // experts of 4096 x 2048 at 252 / 254 / 255 rows 183 / 183 / 184 us with it on 256x256, 177 / 177 / 176 without, at 251 rows
+  // 169 / 174)
+  const bool spills = tiles_l < kNumCu && S * expected_m_tiles(avg, 256) * (p.N / 128) > 1.05 * kNumCu;
+  if (avg >= (tiles_l >= kNumCu ? 40 : 56) && tiles_l >= kNumCu / 2 && !spills) return kTileL;
   return avg >= (tiles_m >= 2 * kNumCu ? 8 : 16) && avg < 64 ? kTileMS : t;
 }
 

@@ -97,8 +97,10 @@ struct RouteHistPlan {
 // measured against the router + two-pass align (one box, cache-cold layers): Qwen3-30B-A3B
 // 32-expert share at 256 and 600 tokens (512 and 1216 cells) 89.0 -> 86.7 and 105.9 -> 101.7
 // us, at 2048 tokens (4096 cells) equal, DeepSeek-V2-Lite 4096 tokens (16384 cells) 611 -> 620 us.
-// Twice as many with workgroups of 16 waves, in place of the separate histogram launch: DeepSeek-V2-Lite
-// 1200 / 4096 tokens 346 / 641 -> 340 / 637 us (with the other changes to the routing kernels).
+// Twice as many with workgroups of 16 waves, in place of the separate histogram launch (layers of tiny experts, which
+// are all routing, us): 64 experts, top 6, 1100 / 2048 / 4096 tokens 33.7 / 34.7 / 38.3 -> 30.0 / 30.9 / 35.2; 32 of 128, top 8,
+// 3000 / 8192 35.1 / 38.3 -> 32.5 / 36.1; all 128, 700 / 2048 37.2 / 39.9 -> 34.3 / 37.3; 32, top 4, 3000 / 8192 32.0 / 40.3 ->
+// 27.9 / 36.6.  Four times as many measured the same there and 44.3 / 49.1 -> 42.5 / 45.8 at 6000 / 8192 tokens over 64.
 constexpr long long kRouteHistMaxCells = 2048;
 
 // Workgroups of 4 waves, or of 8 where that keeps the matrix within bounds (the Qwen3-30B-A3B
